@@ -13,9 +13,9 @@
 //   k_pattern_grad   one lane per sliced-ELLPACK entry position, k columns
 //                    summed in registers, scattered to the CSR position;
 //                    HBM-bound: nnz (4 + 4 + 8) + gathers of X and Y
-//   k_q1_elem_grad   one thread per element: the 8 corner values of x and y
-//                    (zero on Dirichlet nodes) and the integer element
-//                    numerators 36 Khat in constant memory
+//   k_q1_elem_grad   a thread marches up a column of elements: node values of
+//                    x and y (zero on Dirichlet nodes) read once per plane,
+//                    36 Khat diagonal in the sums and differences per axis
 #include <hip/hip_runtime.h>
 
 #include "gcge_hip_internal.h"
@@ -26,6 +26,16 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWave = 64;
+constexpr int kXcds = 8;
+
+// Workgroup b is dispatched to XCD b % 8.  Renumber so that the workgroups of
+// one XCD cover one contiguous range of work items.
+__device__ __forceinline__ int xcd_remap(int bid, int nb)
+{
+    const int q = nb / kXcds, r = nb % kXcds;
+    const int xcd = bid % kXcds, loc = bid / kXcds;
+    return (xcd < r) ? xcd * (q + 1) + loc : r * (q + 1) + (xcd - r) * q + loc;
+}
 
 __global__ __launch_bounds__(kBlock) void k_pattern_grad(int n, int nslices,
                                                         const int *__restrict__ sptr,
@@ -57,9 +67,25 @@ __global__ __launch_bounds__(kBlock) void k_pattern_grad(int n, int nslices,
     }
 }
 
-// 36 * Khat of the unit cube, corners p = 4 ax + 2 ay + az
-__constant__ int c_k36[64];
-
+// Element gradient, bound by the reads of X (8 n k bytes): a thread owns the
+// Z elements ez0 .. ez0 + Z - 1 above one in-plane element (consecutive
+// threads along x, then y) and, for every column, reads the Z + 1 node planes
+// they touch once: 4 (Z + 1) values, all in flight together, instead of 8 per
+// element and operand.  The 8 corner values of an element enter through sums
+// s and differences d along each axis, in which the element matrix is
+// diagonal: per axis x^T k y = d_x d_y and x^T (6 m) y = 3/2 s_x s_y + 1/2
+// d_x d_y, so x^T (36 Khat) y = 9/4 (one difference) + 3/2 (two) + 3/4
+// (three), about 30 operations per element and column instead of 144, and
+// the in-plane half of the transform is shared by the elements below and
+// above a plane.  SPLIT threads of a workgroup share an element column, each
+// taking every SPLIT-th column of X (combined through LDS in a fixed order).
+// SAME: Y is X (read once).  MAP: node numbers go through node_row, once per
+// thread.  Measured (kernel alone, X = Y; before: one thread per element, 16
+// loads and 8 x 8 products): 128^3 elements x 100 columns 1799 -> 617 us (2.7
+// TB/s of X), 64^3 x 20 52 -> 21, 24^3 x 60 46 -> 15, permuted rows at 128^3
+// x 100 17.9 -> 7.0 ms.  Two elements along y per thread (fewer loads each)
+// measured the same, Z = 4 16 % slower at 128^3.
+template <int Z, int SPLIT, bool SAME, bool MAP>
 __global__ __launch_bounds__(kBlock) void k_q1_elem_grad(int E, double scale,
                                                         const double *__restrict__ X, long ldx,
                                                         const double *__restrict__ Y, long ldy,
@@ -67,39 +93,111 @@ __global__ __launch_bounds__(kBlock) void k_q1_elem_grad(int E, double scale,
                                                         const int *__restrict__ node_row,
                                                         double *__restrict__ grad)
 {
-    const long e = (long)blockIdx.x * kBlock + threadIdx.x;
-    const long ne = (long)E * E * E;
-    if (e >= ne) return;
-    const int ex = (int)(e % E), ey = (int)((e / E) % E), ez = (int)(e / ((long)E * E));
-    const int N = E - 1;
-    long node[8];
+    constexpr int EL = kBlock / SPLIT;  // in-plane elements of a workgroup
+    const int N = E - 1, EE = E * E, tiles = (EE + EL - 1) / EL;
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    const int ez0 = blk / tiles * Z;
+    const int part = threadIdx.x / EL, ip = blk % tiles * EL + threadIdx.x % EL;
+    const int ex = ip % E, ey = ip / E;
+    bool ok[4];
+    int off[4];
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-        const int ix = ex + ((p >> 2) & 1), iy = ey + ((p >> 1) & 1), iz = ez + (p & 1);
-        const bool interior = ix >= 1 && ix <= N && iy >= 1 && iy <= N && iz >= 1 && iz <= N;
-        node[p] = interior ? (long)(ix - 1) + (long)N * (iy - 1) + (long)N * N * (iz - 1) : -1;
-        if (node_row && node[p] >= 0) node[p] = node_row[node[p]];  // row of a permuted block
+    for (int q = 0; q < 4; ++q) {
+        const int ix = ex + (q & 1), iy = ey + (q >> 1);
+        ok[q] = ip < EE && ix >= 1 && ix <= N && iy >= 1 && iy <= N;
+        off[q] = ok[q] ? (ix - 1) + N * (iy - 1) : 0;
     }
-    double total = 0.0;
-    for (int c = 0; c < k; ++c) {
-        const double *xc = X + (long)c * ldx, *yc = Y + (long)c * ldy;
-        double xv[8], yv[8];
+    int row[MAP ? Z + 1 : 1][4];
+    if constexpr (MAP) {
 #pragma unroll
-        for (int p = 0; p < 8; ++p) {
-            xv[p] = node[p] >= 0 ? xc[node[p]] : 0.0;
-            yv[p] = node[p] >= 0 ? yc[node[p]] : 0.0;
+        for (int p = 0; p <= Z; ++p) {
+            const int iz = ez0 + p;
+            const bool in = iz >= 1 && iz <= N;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                row[p][q] = in && ok[q] ? node_row[(long)(iz - 1) * N * N + off[q]] : 0;
         }
-        double q = 0.0;
-#pragma unroll
-        for (int p = 0; p < 8; ++p) {
-            double t = 0.0;
-#pragma unroll
-            for (int r = 0; r < 8; ++r) t += (double)c_k36[p * 8 + r] * yv[r];
-            q += xv[p] * t;
-        }
-        total += w[c] * q;
     }
-    grad[e] = scale * total;
+    // corner values of the Z + 1 planes (planes and nodes outside the mesh
+    // read an inside one and count as zero), then the in-plane sums and
+    // differences (x fastest: ss, ds, sd, dd)
+    auto planes = [&](const double *__restrict__ col, double (&t)[Z + 1][4]) {
+#pragma unroll
+        for (int p = 0; p <= Z; ++p) {
+            const double *base = MAP ? col : col + (long)(min(max(ez0 + p, 1), N) - 1) * N * N;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) t[p][q] = base[MAP ? row[MAP ? p : 0][q] : off[q]];
+        }
+#pragma unroll
+        for (int p = 0; p <= Z; ++p) {
+            const bool in = ez0 + p >= 1 && ez0 + p <= N;
+            double v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = in && ok[q] ? t[p][q] : 0.0;
+            const double s0 = v[0] + v[1], d0 = v[1] - v[0], s1 = v[2] + v[3], d1 = v[3] - v[2];
+            t[p][0] = s0 + s1;
+            t[p][1] = d0 + d1;
+            t[p][2] = s1 - s0;
+            t[p][3] = d1 - d0;
+        }
+    };
+    double total[Z];
+#pragma unroll
+    for (int z = 0; z < Z; ++z) total[z] = 0.0;
+    for (int c = part; c < k; c += SPLIT) {
+        double tx[Z + 1][4], ty[SAME ? 1 : Z + 1][4];
+        planes(X + (long)c * ldx, tx);
+        if constexpr (!SAME) planes(Y + (long)c * ldy, ty);
+        const double wc = w[c];
+#pragma unroll
+        for (int z = 0; z < Z; ++z) {
+            double m[8];  // products of the z sums (0..3) and differences (4..7)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double xs = tx[z + 1][q] + tx[z][q], xd = tx[z + 1][q] - tx[z][q];
+                double ys = xs, yd = xd;
+                if constexpr (!SAME) {
+                    ys = ty[z + 1][q] + ty[z][q];
+                    yd = ty[z + 1][q] - ty[z][q];
+                }
+                m[q] = xs * ys;
+                m[4 + q] = xd * yd;
+            }
+            total[z] += wc * (2.25 * (m[1] + m[2] + m[4]) + 1.5 * (m[3] + m[5] + m[6]) + 0.75 * m[7]);
+        }
+    }
+    if constexpr (SPLIT > 1) {
+        __shared__ double red[SPLIT - 1][Z][EL];
+        if (part > 0) {
+#pragma unroll
+            for (int z = 0; z < Z; ++z) red[part - 1][z][threadIdx.x % EL] = total[z];
+        }
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int z = 0; z < Z; ++z)
+#pragma unroll
+            for (int q = 0; q < SPLIT - 1; ++q) total[z] += red[q][z][threadIdx.x];
+    }
+    if (ip < EE) {
+#pragma unroll
+        for (int z = 0; z < Z; ++z)
+            if (ez0 + z < E) grad[(long)(ez0 + z) * EE + ip] = scale * total[z];
+    }
+}
+
+template <int Z, int SPLIT, bool SAME>
+void launch_elem_grad(int E, double scale, const double *X, long ldx, const double *Y, long ldy,
+                      int k, const double *d_w, const int *d_node_row, double *d_grad)
+{
+    constexpr int EL = kBlock / SPLIT;
+    const long nb = ((long)E * E + EL - 1) / EL * ((E + Z - 1) / Z);
+    if (d_node_row)
+        hipLaunchKernelGGL((k_q1_elem_grad<Z, SPLIT, SAME, true>), dim3((unsigned)nb), dim3(kBlock), 0,
+                           state().stream, E, scale, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
+    else
+        hipLaunchKernelGGL((k_q1_elem_grad<Z, SPLIT, SAME, false>), dim3((unsigned)nb), dim3(kBlock), 0,
+                           state().stream, E, scale, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
 }
 
 }  // namespace
@@ -120,28 +218,24 @@ void q1_element_gradient(int E, const double *X, long ldx, const double *Y, long
                          const double *d_w, double *d_grad, const int *d_node_row)
 {
     if (E < 2 || k <= 0) return;
-    static bool uploaded = false;
-    if (!uploaded) {
-        int k36[64];
-        for (int p = 0; p < 8; ++p)
-            for (int q = 0; q < 8; ++q) {
-                const int a[3] = {(p >> 2) & 1, (p >> 1) & 1, p & 1};
-                const int b[3] = {(q >> 2) & 1, (q >> 1) & 1, q & 1};
-                int k1[3], m6[3];
-                for (int d = 0; d < 3; ++d) {
-                    k1[d] = a[d] == b[d] ? 1 : -1;
-                    m6[d] = a[d] == b[d] ? 2 : 1;
-                }
-                k36[p * 8 + q] = k1[0] * m6[1] * m6[2] + m6[0] * k1[1] * m6[2] + m6[0] * m6[1] * k1[2];
-            }
-        HIP_CHECK(hipMemcpyToSymbol(HIP_SYMBOL(c_k36), k36, sizeof(k36)));
-        uploaded = true;
-    }
     const long ne = (long)E * E * E;
     const double h = 1.0 / E;
     ProfScope prof("q1_elem_grad", 16.0 * k * (double)(E - 1) * (E - 1) * (E - 1) + 8.0 * ne);
-    hipLaunchKernelGGL(k_q1_elem_grad, dim3((unsigned)((ne + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                       state().stream, E, h / 36.0, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
+    // eight planes per thread (two operands: four, for the registers) where
+    // that gives six wavefronts per CU, from about E = 90: 617 against 712 us
+    // at 128^3 x 100, 86 against 91 at 97^3 x 33; below, four planes and the
+    // columns of X shared by four threads: 21 against 28 us at 64^3 x 20, 15
+    // against 68 at 24^3 x 60
+    const long waves = ((long)E * E + kWave - 1) / kWave * ((E + 7) / 8);
+    const bool many = waves >= 6L * 256, same = X == Y && ldx == ldy;
+    if (many && same)
+        launch_elem_grad<8, 1, true>(E, h / 36.0, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
+    else if (many)
+        launch_elem_grad<4, 1, false>(E, h / 36.0, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
+    else if (same)
+        launch_elem_grad<4, 4, true>(E, h / 36.0, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
+    else
+        launch_elem_grad<4, 4, false>(E, h / 36.0, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
     HIP_CHECK(hipGetLastError());
 }
 

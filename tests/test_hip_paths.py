@@ -1,0 +1,47 @@
+"""Device kernels at the sizes where their dispatch or their tiles can go
+wrong: tile edges, remainders, the smallest sizes and both sides of a rule
+(GPU).  Tolerances are forward-error bounds: unit roundoff times the number of
+roundings an entry passes through times the sum of its absolute products."""
+import numpy as np
+import pytest
+
+from gcge_old_amd import DeviceMultiVec, adjoint
+from oracle import adjoint as oadj
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(np.float64).eps
+
+
+def _corner_abs_sums(E, X):
+    """sum of |x| over the 8 corners of every element, (E^3, k)"""
+    N = E - 1
+    full = np.zeros((E + 1, E + 1, E + 1, X.shape[1]))
+    full[1:E, 1:E, 1:E] = np.abs(X).reshape(N, N, N, -1)
+    s = sum(full[a:a + E, b:b + E, c:c + E] for a in (0, 1) for b in (0, 1) for c in (0, 1))
+    return s.reshape(E ** 3, -1)
+
+
+@pytest.mark.parametrize("permuted", [False, True])
+@pytest.mark.parametrize("two_blocks", [False, True])
+@pytest.mark.parametrize("E,k", [(2, 1), (3, 2), (9, 5), (17, 3), (33, 9), (92, 2)])
+def test_element_gradient_sizes(E, k, two_blocks, permuted):
+    """Four or eight node planes per thread (from E = 91), columns shared by
+    four threads (k below, above and no multiple of four), planes cut off at
+    the mesh end, one or two blocks, permuted rows."""
+    rng = np.random.default_rng(E * 100 + k)
+    n = (E - 1) ** 3
+    X = rng.standard_normal((n, k))
+    Y = rng.standard_normal((n, k)) if two_blocks else X
+    w = rng.standard_normal(k)
+    print(f"element gradient E={E} k={k} two={two_blocks} permuted={permuted}", flush=True)
+    row = rng.permutation(n) if permuted else None
+    Xr, Yr = np.empty_like(X), np.empty_like(Y)
+    Xr[row if permuted else slice(None)], Yr[row if permuted else slice(None)] = X, Y
+    dX = DeviceMultiVec.from_host(Xr)
+    got = adjoint.q1_kappa_gradient(E, dX, w, Y=DeviceMultiVec.from_host(Yr) if two_blocks else None,
+                                    node_row=row)
+    want = oadj.q1_element_gradient(E, X, w, Y=Y if two_blocks else None)
+    # 36 Khat has entries up to 12 in absolute value, and so have the products
+    # of the transformed corner values; both sides round 16 + k times at most
+    bound = (12.0 / 36.0 / E) * (_corner_abs_sums(E, X) * _corner_abs_sums(E, Y)) @ np.abs(w)
+    assert np.all(np.abs(got - want) <= 2 * (16 + k) * EPS * bound)
