@@ -921,15 +921,11 @@ static void op_mv_lincomb(void **x, void **y, GCGE_INT *start, GCGE_INT *end, do
     check_range(Y, start[1], k, "MultiVecLinearComb");
     if (m <= 0) fail_msg("MultiVecLinearComb: empty input range");
     work_vec(0, (double)m * k, Y->n);  // one axpby per coefficient (src/gcge_ops.c:190-221)
-    // coefficients row by row, zero-padded to the kernel's column group
-    const int g = lincomb_group(k);
-    const int ldct = (k + g - 1) / g * g;
-    std::vector<double> packed((size_t)m * ldct, 0.0);
-    for (int j = 0; j < k; ++j)
-        for (int i = 0; i < m; ++i) packed[(size_t)i * ldct + j] = a[(size_t)j * lda + i];
-    double *d_C = small_buffer(packed.size());
+    std::vector<double> packed;
+    lincomb_pack(a, lda, m, k, packed);
+    double *d_C = small_buffer(packed.size() + kLcSlack);
     upload_async(d_C, packed.data(), packed.size() * sizeof(double));
-    lincomb_dev(Y->n, col_ptr(X, start[0]), X->ld, m, d_C, ldct, beta, col_ptr(Y, start[1]), Y->ld, k);
+    lincomb_dev(Y->n, col_ptr(X, start[0]), X->ld, m, d_C, beta, col_ptr(Y, start[1]), Y->ld, k);
 }
 
 static int ext_lincomb_in_place(void **v, GCGE_INT in, GCGE_INT m, const GCGE_DOUBLE *a,
@@ -942,14 +938,11 @@ static int ext_lincomb_in_place(void **v, GCGE_INT in, GCGE_INT m, const GCGE_DO
     check_range(X, out, k, "MultiVecLinearCombInPlace");
     // the reference's work for the combination and the copy back
     work_vec(0, (double)m * k + k, X->n);
-    const int g = lincomb_group(k);
-    const int ldct = (k + g - 1) / g * g;
-    std::vector<double> packed((size_t)m * ldct, 0.0);
-    for (int j = 0; j < k; ++j)
-        for (int i = 0; i < m; ++i) packed[(size_t)i * ldct + j] = a[(size_t)j * lda + i];
-    double *d_C = small_buffer(packed.size());
+    std::vector<double> packed;
+    lincomb_pack(a, lda, m, k, packed);
+    double *d_C = small_buffer(packed.size() + kLcSlack);
     upload_async(d_C, packed.data(), packed.size() * sizeof(double));
-    lincomb_in_place(X->n, col_ptr(X, in), col_ptr(X, out), X->ld, m, d_C, ldct, k);
+    lincomb_dev(X->n, col_ptr(X, in), X->ld, m, d_C, 0.0, col_ptr(X, out), X->ld, k);
     return 0;
 }
 

@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 namespace gcge_hip {
 
@@ -194,16 +195,15 @@ int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw
 // host G(m x k, ldg) = V^T W
 void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, int k, double *G,
           int ldg, bool sync_result = true);
-// Y = beta Y + V C with Ct = C stored row by row on the device (ldct >= k,
-// a multiple of lincomb_group(k), padding columns zero)
-int lincomb_group(int k);
-void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_Ct, int ldct,
-                 double beta, double *Y, long ldy, int k);
-// Y = V C with Y's columns allowed to overlap V's (same block of columns),
-// for the shapes lincomb_in_place_ok accepts
+// Y = beta Y + V C with the coefficients packed by lincomb_pack on the device,
+// in a buffer with kLcSlack more doubles behind them (read, never used).
+// Y's columns may overlap V's (one block of columns, same rows and leading
+// dimension) for the shapes lincomb_in_place_ok accepts, beta = 0.
+constexpr size_t kLcSlack = 8 * 8 * 64 + 2 * 256;
+void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &out);
+void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
+                 long ldy, int k);
 bool lincomb_in_place_ok(int m, int k);
-void lincomb_in_place(int n, const double *V, double *Y, long ld, int m, const double *d_Ct, int ldct,
-                      int k);
 void axpby(int n, double a, const double *X, long ldx, double b, double *Y, long ldy, int k);
 void swap_cols(int n, double *X, long ldx, double *Y, long ldy, int k);
 // Y(:, ymap[c]) = a[c] X(:, xmap[c]) + b[c] Y(:, ymap[c]), scalars and maps on the device

@@ -15,10 +15,9 @@
 //               output tiles, 32-row steps staged through LDS (transposed),
 //               4x4 register blocks per thread, split over row chunks with a
 //               deterministic second-pass reduction.
-//   lincomb     Y = beta Y + V C: one lane per row holding 8..64 output
-//               columns in registers; the coefficients of one input column
-//               are a wave-uniform contiguous read, so V is read once per
-//               group of up to 64 output columns.
+//   lincomb     Y = beta Y + V C on the matrix cores: a wavefront owns 32 rows
+//               and all output columns of a group, V goes straight to
+//               registers, the coefficients through LDS.
 //   axpby/swap/random/coldots/residual/bcg_*: streaming kernels.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
@@ -1565,189 +1564,196 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const double *__rest
 
 // ---- linear combination --------------------------------------------------------------
 
-// Ct is the coefficient matrix stored row by row (Ct[i*ldct + j] = C(i, j))
-// and padded with zero columns to a multiple of KT, so the KT coefficients a
-// row of V meets are one contiguous, wave-uniform read (scalar loads).  Each
-// lane owns one row and KT accumulators; V is read once per group of KT
-// output columns.
-template <int KT>
-__global__ __launch_bounds__(kBlock) void k_lincomb(int n, const double *__restrict__ V, long ldv,
-                                                   int m, const double *__restrict__ Ct, int ldct,
-                                                   double beta, double *__restrict__ Y, long ldy,
-                                                   int k)
+// Y = beta Y + V C on the matrix cores, computed as Y^T = C^T V^T.  Bound by
+// HBM (8 n (m + k) bytes) up to about 50 output columns, by the FP64 matrix
+// cores beyond.  A wavefront owns 32 rows and every output column of its group
+// (up to 128), so V goes from memory straight to registers, each value read
+// once by one wave: per step of 4 input columns lane l takes rows r0 + 2 (l %
+// 16), + 1 of column 4 step + l / 16 as one 16-byte load (the two rows belong
+// to two row tiles), eight steps ahead of their products.  The columns are NJ
+// tiles of 16 (v_mfma_f64_16x16x4: lane l, component v of the result holds
+// column l / 16 + 4 v) and NQ quads of 4 (v_mfma_f64_4x4x4 with four blocks of
+// four rows: the same V operand, result column l / 16), so no matrix work goes
+// into padding beyond a quad.  The coefficients come packed in operand order
+// (lincomb_pack) and go through two LDS buffers of eight steps shared by the
+// four waves, one barrier per eight steps.  Measured at n = 2 048 383 (before:
+// V and coefficients staged through LDS, columns rounded up to 64 or 128):
+// 300 -> 100 columns 2946 -> 2138 us (57.5 TFLOP/s; a library product of 8192^2
+// reaches 72.5), 100 -> 100 1265 -> 890, 300 -> 33 2001 -> 1262, 60 -> 10 230
+// -> 230 (5.0 TB/s); at n = 250 047, 90 -> 50 92 -> 62, 77 -> 19 49 -> 36.
+typedef double gcge_double2 __attribute__((ext_vector_type(2)));
+constexpr int kLcSteps = 8;  // steps of a stage, at most
+constexpr int kLcCols = 128;  // columns of a group
+
+__device__ __forceinline__ double mfma_quad(double a, double b, double c)
 {
-    const int row = blockIdx.x * kBlock + threadIdx.x;
-    if (row >= n) return;
-    for (int c0 = 0; c0 < k; c0 += KT) {
-        double acc[KT];
-#pragma unroll
-        for (int cc = 0; cc < KT; ++cc) acc[cc] = 0.0;
-        const double *cp = Ct + c0;
-        for (int i = 0; i < m; ++i) {
-            const double v = V[(long)i * ldv + row];
-            const double *ci = cp + (long)i * ldct;
-#pragma unroll
-            for (int cc = 0; cc < KT; ++cc) acc[cc] += v * ci[cc];
-        }
-        const int nc = min(KT, k - c0);
-#pragma unroll
-        for (int cc = 0; cc < KT; ++cc) {
-            if (cc < nc) {
-                double *y = Y + (long)(c0 + cc) * ldy + row;
-                *y = (beta == 0.0) ? acc[cc] : beta * (*y) + acc[cc];
-            }
-        }
-    }
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
 }
 
-// Y = beta Y + V C on the matrix cores, computed as Y^T = C^T V^T with
-// v_mfma_f64_16x16x4f64: a wavefront owns 16 RT rows and 16 TJ output columns
-// (grid y: column groups); per step of 4 input columns the B operand is 16
-// consecutive rows of a V column per lane group (lane l: V(r0 + l % 16,
-// m0 + l / 16)) and the A operand 16 coefficients of a row of Ct; lane l,
-// component v of a tile then holds Y(r0 + l % 16, j0 + l / 16 + 4 v), so 16
-// lanes write 16 consecutive rows of one column.
-template <int TJ, int RT>
-__global__ __launch_bounds__(kBlock) void k_lincomb_mfma(int n, const double *__restrict__ V, long ldv,
-                                                        int m, const double *__restrict__ Ct, int ldct,
-                                                        double beta, double *__restrict__ Y, long ldy,
-                                                        int k)
+template <int NJ, int NQ>
+__global__ __launch_bounds__(kBlock, 4 * NJ + NQ <= 12 ? 4 : 2) void k_lincomb(
+    int n, const double *__restrict__ V, long ldv, int m, const double *__restrict__ Cp, double beta,
+    double *__restrict__ Y, long ldy, int k, int group_cols)
 {
-    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-    const int r0 = (blockIdx.x * (kBlock / kWave) + wid) * 16 * RT;
-    if (r0 >= n) return;
-    const int j0 = blockIdx.y * 16 * TJ;
-    const int kk = lane / 16, li = lane % 16;
-    gcge_double4 acc[TJ][RT];
+    // four steps where the accumulators fill the registers (three instead of two
+    // waves per SIMD: 200 -> 116 columns 2031 -> 1662 us; 300 -> 64 the other way
+    // round, 1497 against 1573)
+    constexpr int S = NJ >= 5 ? kLcSteps / 2 : kLcSteps;
+    constexpr int kStep = NJ * kWave + NQ * 16;  // packed coefficients of a step
+    constexpr int kStage2 = S * kStep / 2;  // pairs of a stage
+    constexpr int kLoads = (kStage2 + kBlock - 1) / kBlock;
+    __shared__ gcge_double2 ldc[2][kLoads * kBlock];
+    const int t = threadIdx.x, lane = t % kWave, kk = lane / 16, li = lane % 16;
+    const int steps = (m + 3) / 4, stages = (steps + S - 1) / S;
+    const gcge_double2 *cp = reinterpret_cast<const gcge_double2 *>(Cp) + (long)blockIdx.y * steps * (kStep / 2) + t;
+    const int r = (blockIdx.x * (kBlock / kWave) + t / kWave) * 32 + 2 * li;
+    // rows past the end repeat, and are not stored; steps past the last
+    // repeat it, and columns past m read column m - 1 and count as zero
+    const double *vp = V + min(r, (n - 1) & ~1) + (long)kk * ldv;
+    const bool in_last = 4 * (steps - 1) + kk < m;
+    const long back = in_last ? 0 : (long)(m - 1 - 4 * (steps - 1) - kk) * ldv;
+    auto vload = [&](int step) {
+        const double *p = vp + (long)(4 * min(step, steps - 1)) * ldv;
+        return *reinterpret_cast<const gcge_double2 *>(step >= steps - 1 ? p + back : p);
+    };
+    gcge_double2 vb[S], pc[kLoads];
 #pragma unroll
-    for (int t = 0; t < TJ; ++t)
+    for (int s = 0; s < S; ++s) vb[s] = vload(s);
+    gcge_double4 acc[2][NJ > 0 ? NJ : 1];
+    double quad[2][NQ > 0 ? NQ : 1];
 #pragma unroll
-        for (int q = 0; q < RT; ++q) acc[t][q] = gcge_double4{0.0, 0.0, 0.0, 0.0};
-    for (int m0 = 0; m0 < m; m0 += 4) {
-        const int mm = m0 + kk;
-        const bool mok = mm < m;
-        double a[TJ], b[RT];
+    for (int q = 0; q < 2; ++q) {
 #pragma unroll
-        for (int t = 0; t < TJ; ++t) {
-            const int j = j0 + t * 16 + li;
-            a[t] = (mok && j < k) ? Ct[(long)mm * ldct + j] : 0.0;
-        }
+        for (int j = 0; j < NJ; ++j) acc[q][j] = gcge_double4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int q = 0; q < RT; ++q) {
-            const int r = r0 + q * 16 + li;
-            b[q] = (mok && r < n) ? V[(long)mm * ldv + r] : 0.0;
-        }
-#pragma unroll
-        for (int t = 0; t < TJ; ++t)
-#pragma unroll
-            for (int q = 0; q < RT; ++q)
-                acc[t][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], b[q], acc[t][q], 0, 0, 0);
+        for (int j = 0; j < NQ; ++j) quad[q][j] = 0.0;
     }
+    auto products = [&](const double *lc, double b0, double b1) {
+        const double *ls = lc + lane, *lq = lc + kk * 4 + lane % 4;
 #pragma unroll
-    for (int t = 0; t < TJ; ++t)
+        for (int j = 0; j < NJ; ++j) {
+            const double a = ls[j * kWave];
+            acc[0][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b0, acc[0][j], 0, 0, 0);
+            acc[1][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, acc[1][j], 0, 0, 0);
+        }
 #pragma unroll
-        for (int q = 0; q < RT; ++q)
+        for (int j = 0; j < NQ; ++j) {
+            const double a = lq[NJ * kWave + j * 16];
+            quad[0][j] = mfma_quad(a, b0, quad[0][j]);
+            quad[1][j] = mfma_quad(a, b1, quad[1][j]);
+        }
+    };
+    // the stage's pairs and what follows them (the buffer has room, kLcSlack)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int j = j0 + t * 16 + kk + 4 * v, r = r0 + q * 16 + li;
-                if (j < k && r < n) {
-                    double *y = Y + (long)j * ldy + r;
-                    *y = (beta == 0.0) ? acc[t][q][v] : beta * (*y) + acc[t][q][v];
-                }
+    for (int u = 0; u < kLoads; ++u) ldc[0][u * kBlock + t] = cp[u * kBlock];
+    lds_barrier();
+    int stage = 0;
+    // stages whose steps are all full columns, without branches
+    for (; stage < (m / 4) / S; ++stage) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) pc[u] = cp[(long)(stage + 1) * kStage2 + u * kBlock];
+        const double *lc = reinterpret_cast<const double *>(ldc[stage & 1]);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            products(lc + s * kStep, vb[s].x, vb[s].y);
+            vb[s] = vload((stage + 1) * S + s);
+        }
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) ldc[(stage + 1) & 1][u * kBlock + t] = pc[u];
+        lds_barrier();
+    }
+    if (stage < stages) {
+        const double *lc = reinterpret_cast<const double *>(ldc[stage & 1]);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int step = stage * S + s;
+            if (step >= steps) break;
+            const bool in = step < steps - 1 || in_last;
+            products(lc + s * kStep, in ? vb[s].x : 0.0, in ? vb[s].y : 0.0);
+        }
+    }
+    const int j0 = blockIdx.y * group_cols;
+    auto put = [&](int j, double y0, double y1) {
+        if (j >= group_cols || j0 + j >= k || r >= n) return;
+        double *y = Y + (long)(j0 + j) * ldy + r;
+        if (r + 1 < n) {
+            double2 *y2 = reinterpret_cast<double2 *>(y);
+            if (beta != 0.0) {
+                const double2 o = *y2;
+                y0 = beta * o.x + y0;
+                y1 = beta * o.y + y1;
             }
+            *y2 = make_double2(y0, y1);
+        } else {
+            *y = beta == 0.0 ? y0 : beta * (*y) + y0;
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) put(16 * j + kk + 4 * v, acc[0][j][v], acc[1][j][v]);
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) put(16 * NJ + 4 * j + kk, quad[0][j], quad[1][j]);
 }
 
-// The same product with V staged through LDS: a workgroup owns 16 RT rows
-// and up to 128 output columns (4 waves x TJW column tiles), so each V value
-// is read from HBM once for all the columns (the wavefront kernel above
-// reads V once per 64 columns, and each wave waits for its own loads).
-// Stages of 16 input columns go through two LDS buffers: the next stage's
-// global loads are issued before the current stage's matrix-core products
-// and written to the other buffer after them, one barrier per stage.  The
-// stage's coefficients C(m0 .. m0+15, jg .. jg+127) go through LDS too: one
-// coalesced load per workgroup instead of one per wavefront and step.
-constexpr int kLcStage = 16;
-template <int TJW, int RT>
-__global__ __launch_bounds__(kBlock, 2) void k_lincomb_lds(int n, const double *__restrict__ V, long ldv,
-                                                          int m, const double *__restrict__ Ct,
-                                                          int ldct, double beta,
-                                                          double *__restrict__ Y, long ldy, int k)
+// The column groups of a combination with k outputs: `groups` of `cols`
+// columns each (the last may have fewer), as nj tiles of 16 and nq quads.
+struct LcShape {
+    int groups, cols, nj, nq;
+};
+inline LcShape lincomb_shape(int k)
 {
-    constexpr int R = 16 * RT;                       // rows per workgroup
-    constexpr int PER = kLcStage * R / kBlock;       // staged values per thread
-    constexpr int CPER = kLcStage * 128 / kBlock;    // staged coefficients per thread
-    __shared__ double lds[2][kLcStage][R];
-    __shared__ double ldc[2][kLcStage][128];
-    const int t = threadIdx.x, lane = t % kWave, wid = t / kWave;
-    const int r0 = blockIdx.x * R;
-    const int jg = blockIdx.y * 128;
-    const int kk = lane / 16, li = lane % 16;
-    gcge_double4 acc[TJW][RT];
-#pragma unroll
-    for (int u = 0; u < TJW; ++u)
-#pragma unroll
-        for (int q = 0; q < RT; ++q) acc[u][q] = gcge_double4{0.0, 0.0, 0.0, 0.0};
-    double pv[PER], pc[CPER];
-    auto load = [&](int m0) {
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int e = t + kBlock * u, c = e / R, r = e % R;
-            pv[u] = (m0 + c < m && r0 + r < n) ? V[(long)(m0 + c) * ldv + r0 + r] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < CPER; ++u) {
-            const int e = t + kBlock * u, i = e / 128, j = jg + e % 128;
-            pc[u] = (m0 + i < m && j < k) ? Ct[(long)(m0 + i) * ldct + j] : 0.0;
-        }
-    };
-    auto stash = [&](int b) {
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int e = t + kBlock * u;
-            lds[b][e / R][e % R] = pv[u];
-        }
-#pragma unroll
-        for (int u = 0; u < CPER; ++u) {
-            const int e = t + kBlock * u;
-            ldc[b][e / 128][e % 128] = pc[u];
-        }
-    };
-    load(0);
-    stash(0);
-    __syncthreads();
-    int buf = 0;
-    for (int m0 = 0; m0 < m; m0 += kLcStage) {
-        const bool more = m0 + kLcStage < m;
-        if (more) load(m0 + kLcStage);
-#pragma unroll
-        for (int st = 0; st < kLcStage / 4; ++st) {
-            double a[TJW], b[RT];
-#pragma unroll
-            for (int u = 0; u < TJW; ++u) a[u] = ldc[buf][4 * st + kk][16 * (wid + 4 * u) + li];
-#pragma unroll
-            for (int q = 0; q < RT; ++q) b[q] = lds[buf][4 * st + kk][16 * q + li];
-#pragma unroll
-            for (int u = 0; u < TJW; ++u)
-#pragma unroll
-                for (int q = 0; q < RT; ++q)
-                    acc[u][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[q], acc[u][q], 0, 0, 0);
-        }
-        if (more) stash(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
+    LcShape s;
+    s.groups = (k + kLcCols - 1) / kLcCols;
+    s.cols = (k + s.groups - 1) / s.groups;
+    s.nj = s.cols / 16;
+    s.nq = (s.cols % 16 + 3) / 4;
+    if (s.nq == 4) {
+        ++s.nj;
+        s.nq = 0;
     }
-#pragma unroll
-    for (int u = 0; u < TJW; ++u)
-#pragma unroll
-        for (int q = 0; q < RT; ++q)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int j = jg + 16 * (wid + 4 * u) + kk + 4 * v, r = r0 + 16 * q + li;
-                if (j < k && r < n) {
-                    double *y = Y + (long)j * ldy + r;
-                    *y = (beta == 0.0) ? acc[u][q][v] : beta * (*y) + acc[u][q][v];
-                }
-            }
+    return s;
+}
+
+template <int NJ>
+void launch_lincomb_q(int nq, dim3 grid, int n, const double *V, long ldv, int m, const double *d_C,
+                      double beta, double *Y, long ldy, int k, int group_cols)
+{
+    hipStream_t st = state().stream;
+#define GCGE_LC(NQ)                                                                               \
+    hipLaunchKernelGGL((k_lincomb<NJ, NQ>), grid, dim3(kBlock), 0, st, n, V, ldv, m, d_C, beta, Y, \
+                       ldy, k, group_cols)
+    if constexpr (NJ > 0) {
+        if (nq == 0) GCGE_LC(0);
+    }
+    if constexpr (NJ < kLcCols / 16) {
+        if (nq == 1) GCGE_LC(1);
+        else if (nq == 2) GCGE_LC(2);
+        else if (nq == 3) GCGE_LC(3);
+    }
+#undef GCGE_LC
+}
+
+void launch_lincomb(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
+                    long ldy, int k)
+{
+    const LcShape s = lincomb_shape(k);
+    const dim3 grid((n + 127) / 128, s.groups);
+#define GCGE_LC(NJ) \
+    case NJ: launch_lincomb_q<NJ>(s.nq, grid, n, V, ldv, m, d_C, beta, Y, ldy, k, s.cols); break
+    switch (s.nj) {
+        GCGE_LC(0);
+        GCGE_LC(1);
+        GCGE_LC(2);
+        GCGE_LC(3);
+        GCGE_LC(4);
+        GCGE_LC(5);
+        GCGE_LC(6);
+        GCGE_LC(7);
+        GCGE_LC(8);
+    }
+#undef GCGE_LC
+    HIP_CHECK(hipGetLastError());
 }
 
 // ---- streaming kernels ------------------------------------------------------------------
@@ -2750,57 +2756,46 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
         for (int i = 0; i < m; ++i) G[(long)j * ldg + i] = h[(long)j * m + i];
 }
 
-int lincomb_group(int k) { return k <= 8 ? 8 : k <= 16 ? 16 : k <= 32 ? 32 : 64; }
-
-// the kernel switches of lincomb_dev (measurement): GCGE_HIP_LINCOMB=fma
-// for the vector kernel, GCGE_HIP_LINCOMB_LDS=0 for the wavefront kernels
-static int lincomb_mode()
+// every column of a block with leading dimension ld starts 16-byte aligned
+template <typename T>
+static bool quad_ok(const T *base, long ld)
 {
-    static const int mode = [] {
-        const char *e = getenv("GCGE_HIP_LINCOMB");
-        return (e && strcmp(e, "fma") == 0) ? 1 : 0;
-    }();
-    return mode;
-}
-static int lincomb_lds_mode()
-{
-    static const int v = [] {
-        const char *e = getenv("GCGE_HIP_LINCOMB_LDS");
-        return e ? atoi(e) : 1;
-    }();
-    return v;
+    return ((uintptr_t)base % 16) == 0 && ((size_t)ld * sizeof(T)) % 16 == 0;
 }
 
-bool lincomb_in_place_ok(int m, int k)
+// C (m x k, leading dimension ldc) in the order the combination reads it: per
+// column group, step of 4 input columns, and tile (4 x 16, output column
+// fastest) or quad (4 x 4), zeros past m and k.  For the library comparison:
+// row by row.
+void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &out)
 {
-    return k > 32 && k <= 128 && m >= 32 && !use_blas() && lincomb_mode() == 0 &&
-           lincomb_lds_mode() != 0;
+    if (use_blas()) {
+        out.resize((size_t)m * k);
+        for (int j = 0; j < k; ++j)
+            for (int i = 0; i < m; ++i) out[(size_t)i * k + j] = C[(size_t)j * ldc + i];
+        return;
+    }
+    const LcShape s = lincomb_shape(k);
+    const int steps = ceil_div(m, 4), per_step = s.nj * kWave + s.nq * 16;
+    out.assign((size_t)s.groups * steps * per_step, 0.0);
+    static_assert(kLcSlack >= kLcSteps * kLcCols / 16 * kWave + 2 * kBlock, "one stage, rounded up");
+    for (int g = 0; g < s.groups; ++g)
+        for (int j = 0; j < std::min(s.cols, k - g * s.cols); ++j) {
+            const double *c = C + (size_t)(g * s.cols + j) * ldc;
+            const bool tile = j < 16 * s.nj;
+            const int w = tile ? 16 : 4;  // columns of the tile or quad
+            double *o = out.data() + (size_t)g * steps * per_step +
+                        (tile ? j / 16 * kWave + j % 16 : s.nj * kWave + (j - 16 * s.nj) / 4 * 16 + j % 4);
+            for (int i = 0; i < m; ++i) o[(size_t)(i / 4) * per_step + i % 4 * w] = c[i];
+        }
 }
 
-// Y = V C where the columns of Y may overlap those of V (one block of
-// columns, same rows and leading dimension).  The LDS-staged kernel loads
-// all m input columns of a workgroup's 128 rows in its stage loop, which
-// ends in a workgroup barrier, and writes those rows only after it; with
-// k <= 128 a single workgroup owns each row block, so the output may
-// overwrite the input (the same kernel, the same arithmetic as the
-// out-of-place call).
-void lincomb_in_place(int n, const double *V, double *Y, long ld, int m, const double *d_Ct, int ldct,
-                      int k)
-{
-    if (n <= 0 || k <= 0) return;
-    if (!lincomb_in_place_ok(m, k)) fail_msg("lincomb_in_place: shape not supported");
-    ProfScope prof("lincomb", 8.0 * (double)n * (m + k));
-    const dim3 g(ceil_div(n, 128), 1), block(kBlock);
-    hipStream_t st = state().stream;
-    if (k > 64)
-        hipLaunchKernelGGL((k_lincomb_lds<2, 8>), g, block, 0, st, n, V, ld, m, d_Ct, ldct, 0.0, Y, ld, k);
-    else
-        hipLaunchKernelGGL((k_lincomb_lds<1, 8>), g, block, 0, st, n, V, ld, m, d_Ct, ldct, 0.0, Y, ld, k);
-    HIP_CHECK(hipGetLastError());
-}
+// the wave that writes a row has read all its inputs, and one group holds
+// every column: the output may overwrite the input
+bool lincomb_in_place_ok(int m, int k) { return m > 0 && k > 0 && k <= kLcCols && !use_blas(); }
 
-void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_Ct, int ldct,
-                 double beta, double *Y, long ldy, int k)
+void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
+                 long ldy, int k)
 {
     if (k <= 0 || n <= 0) return;
     if (m <= 0) {  // empty combination: y = beta y
@@ -2808,55 +2803,17 @@ void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_Ct, in
         return;
     }
     ProfScope prof("lincomb", 8.0 * (double)n * (m + k) + (beta == 0.0 ? 0.0 : 8.0 * (double)n * k));
-    if (use_blas() && m > 16 && k > 16) {
-        // Y = beta Y + V C, C^T stored column-major in d_Ct (leading dimension ldct)
+    if (use_blas()) {
+        // Y = beta Y + V C, C^T stored column-major in d_C (leading dimension k)
         const double one = 1.0;
         if (rocblas_dgemm(blas_handle(), rocblas_operation_none, rocblas_operation_transpose, n, k, m, &one, V,
-                          ldv, d_Ct, ldct, &beta, Y, ldy) != rocblas_status_success)
+                          ldv, d_C, k, &beta, Y, ldy) != rocblas_status_success)
             fail_msg("rocblas_dgemm failed");
         return;
     }
-    const dim3 grid(ceil_div(n, kBlock)), block(kBlock);
-    hipStream_t st = state().stream;
-    const int mode = lincomb_mode();
-    // matrix cores for 9..16 and more than 32 columns: 64 rows x 16 columns
-    // or 32 rows x 64 columns per wavefront; measured on MI355X (n = 250047):
-    // m = 70, k = 10: 27.7 us against 34.1 (vector kernel); m = 90, k = 50:
-    // 113.7 against 136.3; m = 80, k = 30: 57.5 against 47.9, so the vector
-    // kernel keeps 17..32
-    const int lds_mode = lincomb_lds_mode();
-    if (mode == 0 && lds_mode && k > 32 && m >= 32) {
-        // V staged through LDS: 128 rows x up to 128 columns per workgroup
-        const int tjw = std::min(k, 128) > 64 ? 2 : 1;
-        const dim3 g(ceil_div(n, 128), ceil_div(k, 128));
-        if (tjw == 2)
-            hipLaunchKernelGGL((k_lincomb_lds<2, 8>), g, block, 0, st, n, V, ldv, m, d_Ct, ldct, beta, Y,
-                               ldy, k);
-        else
-            hipLaunchKernelGGL((k_lincomb_lds<1, 8>), g, block, 0, st, n, V, ldv, m, d_Ct, ldct, beta, Y,
-                               ldy, k);
-        HIP_CHECK(hipGetLastError());
-        return;
-    }
-    if (mode == 0 && k > 8 && (k <= 16 || k > 32)) {
-        const int wpb = kBlock / kWave;
-        if (k <= 16) {
-            hipLaunchKernelGGL((k_lincomb_mfma<1, 4>), dim3(ceil_div(n, 64 * wpb)), block, 0, st, n, V, ldv, m,
-                               d_Ct, ldct, beta, Y, ldy, k);
-        } else {
-            hipLaunchKernelGGL((k_lincomb_mfma<4, 2>), dim3(ceil_div(n, 32 * wpb), ceil_div(k, 64)), block, 0, st,
-                               n, V, ldv, m, d_Ct, ldct, beta, Y, ldy, k);
-        }
-        HIP_CHECK(hipGetLastError());
-        return;
-    }
-    switch (lincomb_group(k)) {
-    case 8: hipLaunchKernelGGL(k_lincomb<8>, grid, block, 0, st, n, V, ldv, m, d_Ct, ldct, beta, Y, ldy, k); break;
-    case 16: hipLaunchKernelGGL(k_lincomb<16>, grid, block, 0, st, n, V, ldv, m, d_Ct, ldct, beta, Y, ldy, k); break;
-    case 32: hipLaunchKernelGGL(k_lincomb<32>, grid, block, 0, st, n, V, ldv, m, d_Ct, ldct, beta, Y, ldy, k); break;
-    default: hipLaunchKernelGGL(k_lincomb<64>, grid, block, 0, st, n, V, ldv, m, d_Ct, ldct, beta, Y, ldy, k); break;
-    }
-    HIP_CHECK(hipGetLastError());
+    // multivec columns and scratch blocks start on 512-byte boundaries
+    if (!quad_ok(V, ldv) || !quad_ok(Y, ldy)) fail_msg("linear combination: blocks must be 16-byte aligned");
+    launch_lincomb(n, V, ldv, m, d_C, beta, Y, ldy, k);
 }
 
 void axpby(int n, double a, const double *X, long ldx, double b, double *Y, long ldy, int k)
@@ -2930,13 +2887,6 @@ void residual_sq(int n, const double *AX, long ldax, const double *BX, long ldbx
     hipLaunchKernelGGL(k_reduce_rows, dim3(3 * k), dim3(kBlock), 0, state().stream, partial, nbx,
                        d_out);
     HIP_CHECK(hipGetLastError());
-}
-
-// every column of a block with leading dimension ld starts 16-byte aligned
-template <typename T>
-static bool quad_ok(const T *base, long ld)
-{
-    return ((uintptr_t)base % 16) == 0 && ((size_t)ld * sizeof(T)) % 16 == 0;
 }
 
 template <typename PT, typename RT>

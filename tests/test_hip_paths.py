@@ -5,7 +5,7 @@ roundings an entry passes through times the sum of its absolute products."""
 import numpy as np
 import pytest
 
-from gcge_old_amd import DeviceMultiVec, adjoint
+from gcge_old_amd import DeviceMultiVec, _native, adjoint
 from oracle import adjoint as oadj
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +45,42 @@ def test_element_gradient_sizes(E, k, two_blocks, permuted):
     # of the transformed corner values; both sides round 16 + k times at most
     bound = (12.0 / 36.0 / E) * (_corner_abs_sums(E, X) * _corner_abs_sums(E, Y)) @ np.abs(w)
     assert np.all(np.abs(got - want) <= 2 * (16 + k) * EPS * bound)
+
+
+@pytest.mark.parametrize("k", [1, 4, 5, 12, 13, 16, 20, 47, 80, 112, 113, 128, 129, 257])
+@pytest.mark.parametrize("n,m", [(1, 1), (2, 3), (127, 4), (128, 33), (129, 16), (3000, 35)])
+def test_linear_comb_tiles(n, m, k):
+    """Quads and tiles of the output columns, one to three column groups,
+    stages of four and eight steps with and without a rest, a single row and
+    rows that end inside a pair, a wave and a workgroup; NaN in columns next to
+    the ones that are read."""
+    rng = np.random.default_rng(1000 * m + k + n)
+    V = rng.standard_normal((n, m + 2))
+    V[:, 0] = V[:, -1] = np.nan
+    C = np.asfortranarray(rng.standard_normal((m, k)))
+    Y0 = rng.standard_normal((n, k + 1))
+    print(f"linear combination n={n} m={m} k={k}", flush=True)
+    for beta in (0.0, -1.5):
+        dV, dY = DeviceMultiVec.from_host(V), DeviceMultiVec.from_host(Y0)
+        _native.hip().GCGE_HIP_LinearComb(dV.handle, 1, m, _native.as_dptr(C), m, beta, dY.handle, 0, k)
+        got = dY.get()
+        want = V[:, 1:-1] @ C + beta * Y0[:, :k]
+        bound = np.abs(V[:, 1:-1]) @ np.abs(C) + abs(beta) * np.abs(Y0[:, :k])
+        assert np.all(np.abs(got[:, :k] - want) <= 2 * (m + 2) * EPS * bound)
+        np.testing.assert_array_equal(got[:, k:], Y0[:, k:])
+
+
+@pytest.mark.parametrize("m,k", [(5, 3), (40, 20), (130, 100), (70, 128)])
+def test_linear_comb_over_its_input(m, k):
+    """Output columns that overlap the input columns (one block, up to 128
+    output columns): the same bits as into another block."""
+    n = 1003
+    rng = np.random.default_rng(m + k)
+    cols = max(m, k) + 2
+    A = rng.standard_normal((n, cols))
+    C = np.asfortranarray(rng.standard_normal((m, k)))
+    dA, dY = DeviceMultiVec.from_host(A), DeviceMultiVec(n, k)
+    lib = _native.hip()
+    lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dY.handle, 0, k)
+    lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dA.handle, 2, k)
+    np.testing.assert_array_equal(dA.get(2, k), dY.get())
