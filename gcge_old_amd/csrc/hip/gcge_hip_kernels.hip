@@ -11,10 +11,10 @@
 //               of rows (its L2 keeps the band of X that the stencil reuses).
 //               HBM-bound: nnz*(8+4) + n*k*8*2 bytes per launch (float64),
 //               nnz*(4+4) + n*k*4*2 (float32).
-//   gram        V^T W for tall-skinny column-major blocks: 64x64 (or 16-wide)
-//               output tiles, 32-row steps staged through LDS (transposed),
-//               4x4 register blocks per thread, split over row chunks with a
-//               deterministic second-pass reduction.
+//   gram        V^T W for tall-skinny column-major blocks on the matrix cores:
+//               waves own columns of the wider block, which go straight to
+//               registers, the other block goes through LDS; partial results
+//               with a deterministic second-pass reduction.
 //   lincomb     Y = beta Y + V C on the matrix cores: a wavefront owns 32 rows
 //               and all output columns of a group, V goes straight to
 //               registers, the coefficients through LDS.
@@ -1067,66 +1067,6 @@ __global__ __launch_bounds__(kBlock) void k_to_double(size_t len, const float *_
 }
 
 // ---- Gram -----------------------------------------------------------------------
-constexpr int kGramRows = 32;
-
-template <int TM, int TN>
-__global__ __launch_bounds__(kBlock) void k_gram(int n, int rows_per_block,
-                                                const double *__restrict__ V, long ldv, int m,
-                                                const double *__restrict__ W, long ldw, int k,
-                                                double *__restrict__ partial)
-{
-    constexpr int RM = TM / 16, RN = TN / 16;
-    __shared__ double Vs[kGramRows][TM + 1];
-    __shared__ double Ws[kGramRows][TN + 1];
-    const int bx = blockIdx.x;
-    const int i0 = blockIdx.y * TM, j0 = blockIdx.z * TN;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int r_begin = bx * rows_per_block;
-    const int r_end = min(n, r_begin + rows_per_block);
-    double acc[RM][RN];
-#pragma unroll
-    for (int a = 0; a < RM; ++a)
-#pragma unroll
-        for (int b = 0; b < RN; ++b) acc[a][b] = 0.0;
-
-    for (int r0 = r_begin; r0 < r_end; r0 += kGramRows) {
-        // stage V(r0:r0+32, i0:i0+TM) and W(...) transposed into LDS; lanes run
-        // along rows so each column segment is one coalesced read
-        for (int e = threadIdx.x; e < kGramRows * TM; e += kBlock) {
-            const int r = e % kGramRows, c = e / kGramRows;
-            const int gr = r0 + r, gc = i0 + c;
-            Vs[r][c] = (gr < r_end && gc < m) ? V[(long)gc * ldv + gr] : 0.0;
-        }
-        for (int e = threadIdx.x; e < kGramRows * TN; e += kBlock) {
-            const int r = e % kGramRows, c = e / kGramRows;
-            const int gr = r0 + r, gc = j0 + c;
-            Ws[r][c] = (gr < r_end && gc < k) ? W[(long)gc * ldw + gr] : 0.0;
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int r = 0; r < kGramRows; ++r) {
-            double va[RM], wb[RN];
-#pragma unroll
-            for (int a = 0; a < RM; ++a) va[a] = Vs[r][tx + 16 * a];
-#pragma unroll
-            for (int b = 0; b < RN; ++b) wb[b] = Ws[r][ty + 16 * b];
-#pragma unroll
-            for (int a = 0; a < RM; ++a)
-#pragma unroll
-                for (int b = 0; b < RN; ++b) acc[a][b] += va[a] * wb[b];
-        }
-        __syncthreads();
-    }
-    double *out = partial + (long)bx * m * k;
-#pragma unroll
-    for (int a = 0; a < RM; ++a)
-#pragma unroll
-        for (int b = 0; b < RN; ++b) {
-            const int i = i0 + tx + 16 * a, j = j0 + ty + 16 * b;
-            if (i < m && j < k) out[(long)j * m + i] = acc[a][b];
-        }
-}
-
 // Small Gram (m <= MR, k <= KR, MR, KR <= 8): every thread walks rows with
 // stride 256 and keeps the whole m x k block in registers; the block's sums
 // go through wave shuffles and LDS to partial[bx * m * k + j * m + i].
@@ -1176,306 +1116,189 @@ __global__ __launch_bounds__(kBlock) void k_gram_small(int n, int rows_per_block
     }
 }
 
-// Gram for m up to a few hundred and k <= 16 (the W orthonormalisation and
-// Rayleigh-Ritz blocks): wave w of a workgroup owns V columns
-// [(blockIdx.y * 4 + w) * MR, +MR) and every W column (KR >= k); the four
-// waves walk the same rows, so each W row is fetched from memory once per
-// workgroup, and V is read once.  Lanes take consecutive rows.  Each wave
-// reduces its MR x KR block over lanes and writes
-// partial[bx * m * k + j * m + i].
-template <int MR, int KR>
-__global__ __launch_bounds__(kBlock) void k_gram_cols(int n, int rows_per_block,
-                                                     const double *__restrict__ V, long ldv,
-                                                     int m, const double *__restrict__ W,
-                                                     long ldw, int k,
-                                                     double *__restrict__ partial)
-{
-    const int bx = blockIdx.x;
-    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-    const int i0 = (blockIdx.y * (kBlock / kWave) + wid) * MR;
-    if (i0 >= m) return;
-    const int r0 = bx * rows_per_block, r1 = min(n, r0 + rows_per_block);
-    double acc[MR][KR];
-#pragma unroll
-    for (int a = 0; a < MR; ++a)
-#pragma unroll
-        for (int b = 0; b < KR; ++b) acc[a][b] = 0.0;
-    const double *vcol[MR];
-#pragma unroll
-    for (int a = 0; a < MR; ++a) vcol[a] = V + (long)min(i0 + a, m - 1) * ldv;
-    // two rows per lane per step: the loads of both are in flight together
-    int r = r0 + lane;
-    for (; r + kWave < r1; r += 2 * kWave) {
-        double v[2][MR], w[2][KR];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int a = 0; a < MR; ++a) v[h][a] = (i0 + a < m) ? vcol[a][r + h * kWave] : 0.0;
-#pragma unroll
-            for (int b = 0; b < KR; ++b) w[h][b] = b < k ? W[(long)b * ldw + r + h * kWave] : 0.0;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int a = 0; a < MR; ++a)
-#pragma unroll
-                for (int b = 0; b < KR; ++b) acc[a][b] += v[h][a] * w[h][b];
-    }
-    if (r < r1) {
-        double v[MR], w[KR];
-#pragma unroll
-        for (int a = 0; a < MR; ++a) v[a] = (i0 + a < m) ? vcol[a][r] : 0.0;
-#pragma unroll
-        for (int b = 0; b < KR; ++b) w[b] = b < k ? W[(long)b * ldw + r] : 0.0;
-#pragma unroll
-        for (int a = 0; a < MR; ++a)
-#pragma unroll
-            for (int b = 0; b < KR; ++b) acc[a][b] += v[a] * w[b];
-    }
-    double *out = partial + (long)bx * m * k;
-#pragma unroll
-    for (int a = 0; a < MR; ++a)
-#pragma unroll
-        for (int b = 0; b < KR; ++b) {
-            const double t = wave_sum(acc[a][b]);
-            if (lane == 0 && i0 + a < m && b < k) out[(long)b * m + i0 + a] = t;
-        }
-}
-
-// V^T W on the matrix cores (v_mfma_f64_16x16x4f64).  Workgroup (bx, by, bz)
-// takes rows [bx * rows_per_block, ...), V columns [128 by, +128) and W
-// columns [128 bz, +128).  Per stage, 16 rows of those columns go to LDS
-// (row stride MP + KP + 1 doubles: V in the first MP columns, W after),
-// 16 consecutive threads reading one column's 16 consecutive rows; every
-// thread issues all its loads of a stage at once, and the next stage's loads
-// are in flight while the matrix cores work on the current one.  The
-// (16 x 16) output tiles are shared round-robin by the NW waves; each MFMA
-// takes one element of V and one of W per lane from LDS (A: lane l holds
-// Vt[l % 16][l / 16] of the 16 x 4 block, B: W[l / 16][l % 16]), and lane l,
-// component v of the accumulator holds D[l / 16 + 4 v][l % 16] (layout checked
-// against the oracle Gram on the device).  Partials as k_gram.
+typedef double gcge_double2 __attribute__((ext_vector_type(2)));
 typedef double gcge_double4 __attribute__((ext_vector_type(4)));
-constexpr int kGmRows = 16;
-constexpr int kGmCols = 128;
-
-template <int PW, int EPT, int NW>
-__global__ __launch_bounds__(64 * NW) void k_gram_mfma(int n, int rows_per_block,
-                                                     const double *__restrict__ V, long ldv,
-                                                     int m, const double *__restrict__ W,
-                                                     long ldw, int k,
-                                                     double *__restrict__ partial, int bcv, int bcw)
+__device__ __forceinline__ double mfma_quad(double a, double b, double c)
 {
-    extern __shared__ double lds_gm[];
-    const int i_base = blockIdx.y * bcv, j_base = blockIdx.z * bcw;
-    const int mb = min(bcv, m - i_base), kb = min(bcw, k - j_base);
-    const int ti = (mb + 15) / 16, tj = (kb + 15) / 16;
-    const int MP = ti * 16, KP = tj * 16, npairs = ti * tj;
-    const int ld = MP + KP + 1;
-    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-    const int r0 = blockIdx.x * rows_per_block, r1 = min(n, r0 + rows_per_block);
-    const int ncols = MP + KP;
-    // this thread's stage elements: row q, columns c0 + kColStep t
-    constexpr int kColStep = 64 * NW / kGmRows;
-    const int q = threadIdx.x % kGmRows, c0 = threadIdx.x / kGmRows;
-    double buf[EPT];
-    auto load_stage = [&](int rs) {
-        const int r = rs + q;
-#pragma unroll
-        for (int t = 0; t < EPT; ++t) {
-            const int c = c0 + kColStep * t;
-            double v = 0.0;
-            if (r < r1) {
-                if (c < MP) {
-                    if (c < mb) v = V[(long)(i_base + c) * ldv + r];
-                } else if (c - MP < kb) {
-                    v = W[(long)(j_base + c - MP) * ldw + r];
-                }
-            }
-            buf[t] = v;
-        }
-    };
-    gcge_double4 acc[PW];
-#pragma unroll
-    for (int p = 0; p < PW; ++p) acc[p] = gcge_double4{0.0, 0.0, 0.0, 0.0};
-    if (r0 < r1) load_stage(r0);
-    for (int rs = r0; rs < r1; rs += kGmRows) {
-#pragma unroll
-        for (int t = 0; t < EPT; ++t) {
-            const int c = c0 + kColStep * t;
-            if (c < ncols) lds_gm[q * ld + c] = buf[t];
-        }
-        __syncthreads();
-        if (rs + kGmRows < r1) load_stage(rs + kGmRows);
-#pragma unroll
-        for (int kk = 0; kk < kGmRows / 4; ++kk) {
-            const int qa = kk * 4 + lane / 16;
-#pragma unroll
-            for (int p = 0; p < PW; ++p) {
-                const int pair = wid + NW * p;
-                if (pair < npairs) {
-                    const double a = lds_gm[qa * ld + (pair / tj) * 16 + lane % 16];
-                    const double b = lds_gm[qa * ld + MP + (pair % tj) * 16 + lane % 16];
-                    acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[p], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    double *out = partial + (long)blockIdx.x * m * k;
-#pragma unroll
-    for (int p = 0; p < PW; ++p) {
-        const int pair = wid + NW * p;
-        if (pair < npairs) {
-            const int j = j_base + (pair % tj) * 16 + lane % 16;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = i_base + (pair / tj) * 16 + lane / 16 + 4 * v;
-                if (i < i_base + mb && j < j_base + kb) out[(long)j * m + i] = acc[p][v];
-            }
-        }
-    }
+    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
 }
 
-template <int P, int NW>
-void launch_gram_mfma_e(int ept, dim3 grid, size_t lds, int n, int rows, const double *V, long ldv,
-                        int m, const double *W, long ldw, int k, double *partial, int bcv, int bcw)
+// V^T W on the matrix cores (more than eight columns on one side): bound by
+// the FP64 matrix cores (2 n m k operations) above about 50 columns of W, by
+// HBM below.  A workgroup of eight waves holds the whole result (up to 384 x
+// 112 or 256 x 128; wider blocks in several, grid y and z).  Wave w owns the
+// 16-column tiles w, w + 8, w + 16 of V (up to MI of them) against every
+// column of W, so V goes from memory straight to registers, one stage ahead
+// of its products: lane l takes rows 2 (l / 16), + 1 of an eight-row half of
+// column l % 16 as one 16-byte load.  The columns of W, NJ tiles of 16 and a
+// quad of 4 (the 4x4x4 instruction) where up to four are left over, are
+// needed by all waves and go through two LDS buffers in the same operand
+// order, one barrier per stage of 16 G rows.  Waves with one tile less run
+// their own copy of the sweep: a branch around the products made the compiler
+// wait for every outstanding load (2322 us at 300 x 100).  Result: lane l,
+// component v of a tile product holds V column l % 16 against W column l / 16
+// + 4 v, of a quad product W column l / 16; partials: V^T W of each
+// workgroup, element (i, j) of workgroup b at b m k + i si + j sj.
+// Measured at n = 2 048 383 (before: V and W staged through LDS per row
+// range): 300 x 100 3041 -> 2036 us (60.4 TFLOP/s; a library product of 8192^2
+// reaches 72.5), 100 x 100 1324 -> 944, 300 x 16 1882 -> 1141, 50 x 50 622 ->
+// 405; at n = 250 047, 60 x 10 36 -> 26 us (5.4 TB/s), 90 x 50 122 -> 65, 20 x
+// 100 118 -> 42 (the wider block takes the part of V).
+// 16-row groups of a stage, as many as the registers of the loads allow, and
+// workgroups per CU (two within 128 registers)
+__host__ __device__ constexpr int gram_wide_groups(int mi, int nj, int nq)
 {
-    hipStream_t st = state().stream;
-    const dim3 block(64 * NW);
-#define GCGE_GM_LAUNCH(E)                                                                             \
-    hipLaunchKernelGGL((k_gram_mfma<P, E, NW>), grid, block, lds, st, n, rows, V, ldv, m, W, ldw, k, \
-                       partial, bcv, bcw)
-    if (ept <= 2) GCGE_GM_LAUNCH(2);
-    else if (ept <= 4) GCGE_GM_LAUNCH(4);
-    else if (ept <= 8) GCGE_GM_LAUNCH(8);
-    else GCGE_GM_LAUNCH(16);
-#undef GCGE_GM_LAUNCH
+    return mi == 2 && mi * (4 * nj + nq) <= 16 ? 4 : mi * (4 * nj + nq) <= 52 ? 2 : 1;
+}
+__host__ __device__ constexpr int gram_wide_blocks(int mi, int nj, int nq)
+{
+    return 2 * mi * (4 * nj + nq) + 8 * gram_wide_groups(mi, nj, nq) * mi + 4 * (nj + nq) <= 96 ? 2 : 1;
 }
 
-// tile pairs per wave: 1, 2 or 8 (the 4-pair instance keeps its
-// accumulators in VGPRs and drops to one or two waves per SIMD; the 8-pair
-// one does not); NW = 4 or 8 waves per workgroup; output blocks of bcv x bcw
-void launch_gram_mfma(int nw, int pw, int ept, dim3 grid, size_t lds, int n, int rows,
-                      const double *V, long ldv, int m, const double *W, long ldw, int k,
-                      double *partial, int bcv, int bcw)
+template <int MI, int NJ, int NQ>
+__global__ __launch_bounds__(512, gram_wide_blocks(MI, NJ, NQ)) void k_gram_wide(
+    int n, const double *__restrict__ V, long ldv, int m,
+    const double *__restrict__ W, long ldw, int k, double *__restrict__ partial, int mc, int kc,
+    int si, int sj)
 {
-#define GCGE_GM_ARGS ept, grid, lds, n, rows, V, ldv, m, W, ldw, k, partial, bcv, bcw
-    if (nw == 8) {
-        if (pw <= 1) launch_gram_mfma_e<1, 8>(GCGE_GM_ARGS);
-        else if (pw <= 2) launch_gram_mfma_e<2, 8>(GCGE_GM_ARGS);
-        else launch_gram_mfma_e<8, 8>(GCGE_GM_ARGS);
-    } else {
-        if (pw <= 1) launch_gram_mfma_e<1, 4>(GCGE_GM_ARGS);
-        else if (pw <= 2) launch_gram_mfma_e<2, 4>(GCGE_GM_ARGS);
-        else launch_gram_mfma_e<8, 4>(GCGE_GM_ARGS);
-    }
-#undef GCGE_GM_ARGS
-}
-
-// V^T W on the matrix cores for the wide projection blocks (64 <= m <= 128
-// MI, 64 <= k <= 16 NJ): one workgroup of eight waves holds the whole m x k
-// result of its row range, so V and W are read from HBM once.  Wave w owns
-// the output row tiles w, w + 8, w + 16 (up to MI of them) against every
-// column tile; per step of 4 rows it reads its column operands once and its
-// row operands once from LDS for up to MI x NJ matrix-core products.  Stages
-// of 16 rows go through two LDS buffers (row stride kGlLd, V columns first):
-// the next stage's global loads are issued before the current stage's
-// products and written to the other buffer after them, one barrier per
-// stage.  MFMA operand and accumulator layout as in k_gram_mfma; partials as
-// k_gram (one m x k block per row range).
-constexpr int kGlStage = 16;
-
-template <int MI, int NJ>
-__global__ __launch_bounds__(512) void k_gram_lds(int n, int rows_per_block,
-                                                  const double *__restrict__ V, long ldv, int m,
-                                                  const double *__restrict__ W, long ldw, int k,
-                                                  double *__restrict__ partial)
-{
-    constexpr int kLd = MI * 128 + NJ * 16 + 1;  // odd: rows start in different banks
-    constexpr int kPass = 512 / kGlStage;        // columns staged per pass
-    constexpr int EPT = (MI * 128 + NJ * 16 + kPass - 1) / kPass;
-    __shared__ double lds[2][kGlStage][kLd];
-    const int ti = (m + 15) / 16, tj = (k + 15) / 16;
-    const int MP = ti * 16, ncols = MP + tj * 16;
-    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-    const int li = lane % 16, lq = lane / 16;
-    const int r0 = blockIdx.x * rows_per_block, r1 = min(n, r0 + rows_per_block);
-    const int q = threadIdx.x % kGlStage, c0 = threadIdx.x / kGlStage;
-    double buf[EPT];
-    auto load = [&](int rs) {
-        const int r = rs + q;
-#pragma unroll
-        for (int u = 0; u < EPT; ++u) {
-            const int c = c0 + kPass * u;
-            double v = 0.0;
-            if (r < r1) {
-                if (c < MP) {
-                    if (c < m) v = V[(long)c * ldv + r];
-                } else if (c - MP < k) {
-                    v = W[(long)(c - MP) * ldw + r];
-                }
-            }
-            buf[u] = v;
-        }
-    };
-    auto stash = [&](int b) {
-#pragma unroll
-        for (int u = 0; u < EPT; ++u) {
-            const int c = c0 + kPass * u;
-            if (c < ncols) lds[b][q][c] = buf[u];
-        }
-    };
-    gcge_double4 acc[MI][NJ];
+    constexpr int G = gram_wide_groups(MI, NJ, NQ);    // 16-row groups of a stage
+    constexpr int kHalf = NJ * kWave + NQ * 16;        // pairs of W per eight-row half
+    constexpr int kPairs = 2 * G * kHalf;
+    constexpr int kLoads = (kPairs + 511) / 512;
+    __shared__ gcge_double2 lds[2][kLoads * 512];
+    const int t = threadIdx.x, lane = t % kWave, wid = t / kWave, li = lane % 16, lq = lane / 16;
+    const int i0 = blockIdx.y * mc, j0 = blockIdx.z * kc;
+    const int mb = min(mc, m - i0), kb = min(kc, k - j0);
+    const int ti = (mb + 15) / 16;
+    // stages first, first + nbx, ...: the workgroups at work read neighbouring
+    // rows (the pages of every column, DRAM rows)
+    const int nbx = gridDim.x, first = blockIdx.x, r0 = first * 16 * G;
+    // columns past the end repeat the last one; their products are not stored
+    const double *vp[MI], *wp[kLoads];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
+        vp[i] = V + (long)(i0 + min(16 * (wid + 8 * i) + li, mb - 1)) * ldv + r0 + 2 * lq;
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+        const int e = u * 512 + t, h = min(e / kHalf, 2 * G - 1), f = e % kHalf;
+        const int q = f - NJ * kWave;  // quads follow the tiles: 16 pairs each
+        const int col = q < 0 ? f / kWave * 16 + f % 16 : NJ * 16 + q / 16 * 4 + q % 4;
+        const int kk = q < 0 ? f % kWave / 16 : q % 16 / 4;
+        wp[u] = W + (long)(j0 + min(col, kb - 1)) * ldw + r0 + 8 * h + 2 * kk;
+    }
+    gcge_double4 acc[MI][NJ];
+    double quad[MI][NQ > 0 ? NQ : 1];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = gcge_double4{0.0, 0.0, 0.0, 0.0};
-    if (r0 < r1) {
-        load(r0);
-        stash(0);
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) quad[i][j] = 0.0;
     }
-    __syncthreads();
-    int b = 0;
-    for (int rs = r0; rs < r1; rs += kGlStage) {
-        const bool more = rs + kGlStage < r1;
-        if (more) load(rs + kGlStage);
-        // NJ is the number of 16-column tiles of W (the launch picks the
-        // instance), so the products of a row tile run without branches
+    // row offsets of a load are constant within a stage, whose first row the
+    // pointers hold
+    auto load2 = [](const double *p) { return *reinterpret_cast<const gcge_double2 *>(p); };
+    const int stages = n / (16 * G), rest = n % (16 * G);
+    const int mine = first < stages ? (stages - first + nbx - 1) / nbx : 0;
+    // the row sweep of a wave with M tiles of V, without branches
+    auto sweep = [&](auto tiles) {
+        constexpr int M = decltype(tiles)::value, MA = M > 0 ? M : 1;
+        gcge_double2 va[2 * G][MA], pw[kLoads];
+        auto products = [&](const gcge_double2 *lw, int h) {
+            if constexpr (M > 0) {
+                gcge_double2 bt[NJ], bq[NQ > 0 ? NQ : 1];
 #pragma unroll
-        for (int kk = 0; kk < kGlStage / 4; ++kk) {
-            const int qa = 4 * kk + lq;
-            double bw[NJ];
+                for (int j = 0; j < NJ; ++j) bt[j] = lw[h * kHalf + j * kWave + lane];
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) bw[j] = lds[b][qa][MP + 16 * j + li];
+                for (int j = 0; j < NQ; ++j) bq[j] = lw[h * kHalf + NJ * kWave + j * 16 + lq * 4 + lane % 4];
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                const int it = wid + 8 * i;
-                if (it < ti) {
-                    const double a = lds[b][qa][16 * it + li];
+                for (int i = 0; i < M; ++i)
 #pragma unroll
-                    for (int j = 0; j < NJ; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bw[j], acc[i][j], 0, 0, 0);
-                }
+                    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+                            acc[i][j] =
+                                __builtin_amdgcn_mfma_f64_16x16x4f64(bt[j][c], va[h][i][c], acc[i][j], 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < NQ; ++j) quad[i][j] = mfma_quad(bq[j][c], va[h][i][c], quad[i][j]);
+                    }
             }
+        };
+        if (mine > 0) {
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) lds[0][u * 512 + t] = load2(wp[u]);
+#pragma unroll
+            for (int h = 0; h < 2 * G; ++h)
+#pragma unroll
+                for (int i = 0; i < M; ++i) va[h][i] = load2(vp[i] + 8 * h);
         }
-        if (more) stash(b ^ 1);
-        __syncthreads();
-        b ^= 1;
-    }
+        lds_barrier();
+        for (int st = 0; st < mine; ++st) {
+            // after the last stage its rows again (never used)
+            const long next = st + 1 < mine ? (long)nbx * 16 * G : 0;
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                wp[u] += next;
+                pw[u] = load2(wp[u]);
+            }
+#pragma unroll
+            for (int i = 0; i < M; ++i) vp[i] += next;
+            const gcge_double2 *lw = lds[st & 1];
+#pragma unroll
+            for (int h = 0; h < 2 * G; ++h) {
+                products(lw, h);
+#pragma unroll
+                for (int i = 0; i < M; ++i) va[h][i] = load2(vp[i] + 8 * h);
+            }
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) lds[(st + 1) & 1][u * 512 + t] = pw[u];
+            lds_barrier();
+        }
+        if (rest > 0 && first == stages % nbx) {
+            // rows past the end count as zero on both sides; loads stay inside
+            const int base = n - rest, last = (n - 1) & ~1;
+            const long adv = (long)base - (r0 + (long)max(mine - 1, 0) * nbx * 16 * G);
+            auto tail = [&](const double *p, int off) {
+                const int r = base + off;  // first row of the pair
+                const gcge_double2 v = load2(p + adv + (min(r, last) - r));
+                return gcge_double2{r < n ? v[0] : 0.0, r + 1 < n ? v[1] : 0.0};
+            };
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                const int e = u * 512 + t, h = min(e / kHalf, 2 * G - 1), f = e % kHalf;
+                const int kk = f < NJ * kWave ? f % kWave / 16 : (f - NJ * kWave) % 16 / 4;
+                lds[0][e] = tail(wp[u], 8 * h + 2 * kk);
+            }
+#pragma unroll
+            for (int h = 0; h < 2 * G; ++h)
+#pragma unroll
+                for (int i = 0; i < M; ++i) va[h][i] = tail(vp[i] + 8 * h, 8 * h + 2 * lq);
+            lds_barrier();
+#pragma unroll
+            for (int h = 0; h < 2 * G; ++h) products(lds[0], h);
+        }
+    };
+    if (__builtin_amdgcn_readfirstlane(wid) + 8 * (MI - 1) < ti)
+        sweep(std::integral_constant<int, MI>{});
+    else
+        sweep(std::integral_constant<int, MI - 1>{});
     double *out = partial + (long)blockIdx.x * m * k;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-        const int it = wid + 8 * i;
-        if (it >= ti) continue;
+        const int c = 16 * (wid + 8 * i) + li;
+        if (c >= mb) continue;
+        double *o = out + (long)(i0 + c) * si;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int col = 16 * j + li;
-            if (j >= tj || col >= k) continue;
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int row = 16 * it + lq + 4 * v;
-                if (row < m) out[(long)col * m + row] = acc[i][j][v];
+                const int d = 16 * j + lq + 4 * v;
+                if (d < kb) o[(long)(j0 + d) * sj] = acc[i][j][v];
             }
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {
+            const int d = 16 * NJ + 4 * j + lq;
+            if (d < kb) o[(long)(j0 + d) * sj] = quad[i][j];
         }
     }
 }
@@ -1491,42 +1314,69 @@ static int num_cus()
     return s.cus;
 }
 
-// the k_gram_lds instance for an m x k block, false when none covers it
-static bool launch_gram_lds(int nbx, int n, int rows, const double *V, long ldv, int m, const double *W,
-                     long ldw, int k, double *partial)
+// The result blocks of k_gram_wide for an m x k product: gy x gz blocks of mc
+// x kc columns, mi tiles of V per wave, nj tiles of W and a quad where up to
+// four columns are left over.
+struct GramShape {
+    int gy, gz, mc, kc, mi, nj, nq;
+};
+inline GramShape gram_wide_shape(int m, int k)
 {
-    const int ti = (m + 15) / 16, tj = (k + 15) / 16;
-    const int mi = (ti + 7) / 8;
-    hipStream_t st = state().stream;
-#define GCGE_GL(MI, NJ)                                                                                  \
-    hipLaunchKernelGGL((k_gram_lds<MI, NJ>), dim3(nbx), dim3(512), 0, st, n, rows, V, ldv, m, W, ldw, k, \
-                       partial)
-#define GCGE_GL_MI(NJ)                       \
-    do {                                     \
-        if (mi == 1) GCGE_GL(1, NJ);         \
-        else if (mi == 2) GCGE_GL(2, NJ);    \
-        else if (mi == 3) GCGE_GL(3, NJ);    \
-        else return false;                   \
-    } while (0)
-    // one instance per W tile count: no masked products
-    switch (tj) {
-    case 1: GCGE_GL_MI(1); break;
-    case 2: GCGE_GL_MI(2); break;
-    case 3: GCGE_GL_MI(3); break;
-    case 4: GCGE_GL_MI(4); break;
-    case 5: GCGE_GL_MI(5); break;
-    case 6: GCGE_GL_MI(6); break;
-    case 7: GCGE_GL_MI(7); break;
-    case 8:
-        if (mi == 1) GCGE_GL(1, 8);
-        else if (mi == 2) GCGE_GL(2, 8);
-        else return false;
-        break;
-    default: return false;
+    GramShape g;
+    g.gz = (k + 127) / 128;
+    g.kc = (k + g.gz - 1) / g.gz;
+    g.nj = std::max(1, g.kc / 16);
+    g.nq = g.kc > 16 ? (g.kc % 16 + 3) / 4 : 0;
+    if (g.nq > 1 || (g.nq > 0 && g.nj == 7)) {
+        ++g.nj;
+        g.nq = 0;
     }
-#undef GCGE_GL_MI
-#undef GCGE_GL
-    return true;
+    const int ti = (m + 15) / 16, most = g.nj == 8 ? 16 : 24;  // accumulators of 3 x 8 tiles do not fit
+    g.gy = (ti + most - 1) / most;
+    g.mc = (ti + g.gy - 1) / g.gy * 16;
+    g.mi = (g.mc / 16 + 7) / 8;
+    return g;
+}
+
+template <int MI, int NJ>
+void launch_gram_wide_q(const GramShape &g, dim3 grid, int n, const double *V, long ldv, int m,
+                        const double *W, long ldw, int k, double *partial, int si, int sj)
+{
+    hipStream_t st = state().stream;
+#define GCGE_GW(NQ)                                                                                       \
+    hipLaunchKernelGGL((k_gram_wide<MI, NJ, NQ>), grid, dim3(512), 0, st, n, V, ldv, m, W, ldw, k, partial, \
+                       g.mc, g.kc, si, sj)
+    if (g.nq == 0) GCGE_GW(0);
+    if constexpr (NJ < 7) {
+        if (g.nq == 1) GCGE_GW(1);
+    }
+#undef GCGE_GW
+}
+
+void launch_gram_wide(const GramShape &g, int nbx, int n, const double *V, long ldv, int m, const double *W,
+                      long ldw, int k, double *partial, int si, int sj)
+{
+    const dim3 grid(nbx, g.gy, g.gz);
+#define GCGE_GW_MI(MI, NJ) launch_gram_wide_q<MI, NJ>(g, grid, n, V, ldv, m, W, ldw, k, partial, si, sj)
+#define GCGE_GW(NJ)                          \
+    case NJ:                                 \
+        if (g.mi == 1) GCGE_GW_MI(1, NJ);    \
+        else if (g.mi == 2) GCGE_GW_MI(2, NJ); \
+        else if constexpr (NJ < 8) GCGE_GW_MI(3, NJ); \
+        break
+    switch (g.nj) {
+        GCGE_GW(1);
+        GCGE_GW(2);
+        GCGE_GW(3);
+        GCGE_GW(4);
+        GCGE_GW(5);
+        GCGE_GW(6);
+        GCGE_GW(7);
+        GCGE_GW(8);
+    }
+#undef GCGE_GW
+#undef GCGE_GW_MI
+    HIP_CHECK(hipGetLastError());
 }
 
 // out[e] = sum_b partial[b * stride + e], e < count.  A block owns OUTS
@@ -1581,14 +1431,8 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const double *__rest
 // 300 -> 100 columns 2946 -> 2138 us (57.5 TFLOP/s; a library product of 8192^2
 // reaches 72.5), 100 -> 100 1265 -> 890, 300 -> 33 2001 -> 1262, 60 -> 10 230
 // -> 230 (5.0 TB/s); at n = 250 047, 90 -> 50 92 -> 62, 77 -> 19 49 -> 36.
-typedef double gcge_double2 __attribute__((ext_vector_type(2)));
 constexpr int kLcSteps = 8;  // steps of a stage, at most
 constexpr int kLcCols = 128;  // columns of a group
-
-__device__ __forceinline__ double mfma_quad(double a, double b, double c)
-{
-    return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
-}
 
 template <int NJ, int NQ>
 __global__ __launch_bounds__(kBlock, 4 * NJ + NQ <= 12 ? 4 : 2) void k_lincomb(
@@ -2570,6 +2414,13 @@ static rocblas_handle blas_handle()
     return h;
 }
 
+// every column of a block with leading dimension ld starts 16-byte aligned
+template <typename T>
+static bool quad_ok(const T *base, long ld)
+{
+    return ((uintptr_t)base % 16) == 0 && ((size_t)ld * sizeof(T)) % 16 == 0;
+}
+
 // The row ranges of a Gram launch: as many as `want`, or fewer when the
 // caller's partial buffer (cap doubles, 0: the backend's grown buffer)
 // cannot hold that many m x k blocks; rows per range rounded up to `gran`.
@@ -2624,111 +2475,23 @@ int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw
         reduce_partials(partial, mk, nbx, mk, d_out);
         return nbx;
     }
-    static const int gram_mode = [] {
-        const char *e = getenv("GCGE_HIP_GRAM");  // "fma": the vector-FMA kernels (measurement)
-        return (e && strcmp(e, "fma") == 0) ? 1 : 0;
-    }();
-    // smallest m for the whole-block kernel, any k (GCGE_HIP_GRAM_LDS; 0: the
-    // k_gram_mfma blocks only, for measurement).  Measured at n = 2 048 383
-    // (wall time of the call): 300 x 48 1.81 against 2.81 ms, 300 x 16 1.89
-    // against 2.03, 200 x 8 0.87 against 1.39, 100 x 24 0.65 against 0.88;
-    // at n = 250 047, 60 x 10 took 68 against 57 us, so small m stay on the
-    // other kernels
-    static const int gram_lds_min = [] {
-        const char *e = getenv("GCGE_HIP_GRAM_LDS");
-        return e ? atoi(e) : 64;
-    }();
-    const int gti = ceil_div(m, 16), gtj = ceil_div(k, 16);
-    if (gram_mode == 0 && gram_lds_min > 0 && m >= gram_lds_min &&
-        ((gtj <= 7 && gti <= 24) || (gtj == 8 && gti <= 16))) {
-        // one workgroup per CU (eight waves, up to 127 KiB of LDS), the whole
-        // m x k block each, about 500 stages of 16 rows per workgroup at 128^3
-        nbx = gram_ranges(n, std::min(ceil_div(n, 4 * kGlStage), num_cus()), mk, partial_cap, kGlStage,
-                          &rows);
-        if (!partial) partial = partial_buffer((size_t)nbx * mk);
-        {
-            ProfScope prof(pname, gbytes);
-            if (!launch_gram_lds(nbx, n, rows, V, ldv, m, W, ldw, k, partial)) fail_msg("k_gram_lds shape");
-            HIP_CHECK(hipGetLastError());
-        }
-        ProfScope prof(rname);
-        reduce_partials(partial, mk, nbx, mk, d_out);
-        return nbx;
-    }
-    if (gram_mode == 0) {
-        // matrix cores: 128 x 128 output blocks (grid y, z), tile pairs shared
-        // by four or eight waves (one block of up to 304 x 128 outputs, W read
-        // once, measured slower at 300 x 100: 5.85 against 4.77 ms)
-        const int bcv = kGmCols, bcw = kGmCols;
-        const int gy = ceil_div(m, bcv), gz = ceil_div(k, bcw);
-        const int ti = ceil_div(std::min(m, bcv), 16), tj = ceil_div(std::min(k, bcw), 16);
-        // eight waves per workgroup beyond 32 output tiles (four would hold 9..16
-        // accumulator tiles each and run at one wave per SIMD)
-        const int nw = ti * tj > 32 ? 8 : 4;
-        const int pw = ceil_div(ti * tj, nw);
-        const int ncols = 16 * (ti + tj);
-        const int ept = ceil_div(kGmRows * ncols, 64 * nw);
-        const size_t lds = (size_t)kGmRows * (ncols + 1) * sizeof(double);
-        // about four workgroups per CU in all, at least two stages each, and
-        // partials of at most a tenth of the input bytes (the reduction pass
-        // reads them all)
-        const long cap_parts = std::max(1L, (long)n * (m + k) / (10L * mk));
-        int want = std::max(1, std::min(ceil_div(n, 2 * kGmRows), std::max(1, 1024 / (gy * gz))));
-        want = (int)std::min<long>(want, cap_parts);
-        nbx = gram_ranges(n, want, mk, partial_cap, kGmRows, &rows);
-        if (!partial) partial = partial_buffer((size_t)nbx * mk);
-        {
-            ProfScope prof(pname, gbytes);
-            dim3 grid(nbx, gy, gz);
-            launch_gram_mfma(nw, pw, ept, grid, lds, n, rows, V, ldv, m, W, ldw, k, partial, bcv, bcw);
-            HIP_CHECK(hipGetLastError());
-        }
-        ProfScope prof(rname);
-        reduce_partials(partial, mk, nbx, mk, d_out);
-        return nbx;
-    }
-    if (k <= 16) {
-        // column-block register path: 8 x 8 or 4 x 16 accumulators per lane
-        const int MR = k <= 8 ? 8 : 4;
-        const int colblocks = ceil_div(m, MR);
-        const int gy = ceil_div(colblocks, kBlock / kWave);
-        nbx = gram_ranges(n, std::min(ceil_div(n, 4 * kWave), std::max(1, 1024 / gy)), mk, partial_cap, 1,
-                          &rows);
-        if (!partial) partial = partial_buffer((size_t)nbx * mk);
-        {
-            ProfScope prof(pname, gbytes);
-            if (k <= 8)
-                hipLaunchKernelGGL((k_gram_cols<8, 8>), dim3(nbx, gy), dim3(kBlock), 0, s.stream, n, rows, V,
-                                   ldv, m, W, ldw, k, partial);
-            else
-                hipLaunchKernelGGL((k_gram_cols<4, 16>), dim3(nbx, gy), dim3(kBlock), 0, s.stream, n, rows, V,
-                                   ldv, m, W, ldw, k, partial);
-            HIP_CHECK(hipGetLastError());
-        }
-        ProfScope prof(rname);
-        reduce_partials(partial, mk, nbx, mk, d_out);
-        return nbx;
-    }
-    const bool wide_m = m > 16, wide_k = k > 16;
-    const int TM = wide_m ? 64 : 16, TN = wide_k ? 64 : 16;
-    const int tm = ceil_div(m, TM), tn = ceil_div(k, TN);
-    const int tiles = tm * tn;
-    // about two workgroups per CU over all tiles, at least 256 rows each
-    nbx = gram_ranges(n, std::min(ceil_div(n, kBlock), std::max(1, 512 / tiles)), mk, partial_cap,
-                      kGramRows, &rows);
+    // multivec columns and scratch blocks start on 512-byte boundaries
+    if (!quad_ok(V, ldv) || !quad_ok(W, ldw)) fail_msg("Gram product: blocks must be 16-byte aligned");
+    // the wider block is the one whose columns the waves share out
+    const bool swap = m < k;
+    const double *A = swap ? W : V, *B = swap ? V : W;
+    const long lda = swap ? ldw : ldv, ldb = swap ? ldv : ldw;
+    const int ma = swap ? k : m, kb = swap ? m : k;
+    const GramShape g = gram_wide_shape(ma, kb);
+    // the workgroups the CUs hold, at least two stages each (at n = 12 167, 50 x
+    // 50: 10.5 us against 12.5 with one, 13.3 with four)
+    const int stage = 16 * gram_wide_groups(g.mi, g.nj, g.nq);
+    const int want = std::max(1, num_cus() * gram_wide_blocks(g.mi, g.nj, g.nq) / (g.gy * g.gz));
+    nbx = gram_ranges(n, std::min(ceil_div(n, 2 * stage), want), mk, partial_cap, 1, &rows);
     if (!partial) partial = partial_buffer((size_t)nbx * mk);
     {
         ProfScope prof(pname, gbytes);
-        dim3 grid(nbx, tm, tn);
-        if (wide_m && wide_k)
-            hipLaunchKernelGGL((k_gram<64, 64>), grid, dim3(kBlock), 0, s.stream, n, rows, V, ldv, m, W, ldw, k, partial);
-        else if (wide_m)
-            hipLaunchKernelGGL((k_gram<64, 16>), grid, dim3(kBlock), 0, s.stream, n, rows, V, ldv, m, W, ldw, k, partial);
-        else if (wide_k)
-            hipLaunchKernelGGL((k_gram<16, 64>), grid, dim3(kBlock), 0, s.stream, n, rows, V, ldv, m, W, ldw, k, partial);
-        else
-            hipLaunchKernelGGL((k_gram<16, 16>), grid, dim3(kBlock), 0, s.stream, n, rows, V, ldv, m, W, ldw, k, partial);
-        HIP_CHECK(hipGetLastError());
+        launch_gram_wide(g, nbx, n, A, lda, ma, B, ldb, kb, partial, swap ? m : 1, swap ? 1 : m);
     }
     ProfScope prof(rname);
     reduce_partials(partial, mk, nbx, mk, d_out);
@@ -2754,13 +2517,6 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
     HIP_CHECK(hipStreamSynchronize(s.stream));
     for (int j = 0; j < k; ++j)
         for (int i = 0; i < m; ++i) G[(long)j * ldg + i] = h[(long)j * m + i];
-}
-
-// every column of a block with leading dimension ld starts 16-byte aligned
-template <typename T>
-static bool quad_ok(const T *base, long ld)
-{
-    return ((uintptr_t)base % 16) == 0 && ((size_t)ld * sizeof(T)) % 16 == 0;
 }
 
 // C (m x k, leading dimension ldc) in the order the combination reads it: per

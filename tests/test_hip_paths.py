@@ -84,3 +84,22 @@ def test_linear_comb_over_its_input(m, k):
     lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dY.handle, 0, k)
     lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dA.handle, 2, k)
     np.testing.assert_array_equal(dA.get(2, k), dY.get())
+
+
+@pytest.mark.parametrize("m,k", [(9, 1), (1, 9), (17, 5), (16, 100), (48, 20), (129, 33), (113, 113),
+                                 (300, 114), (257, 127), (400, 10), (30, 390), (130, 260)])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 65, 1000])
+def test_gram_tiles(n, m, k):
+    """One to three tiles of the wider block per wave with waves left over,
+    tiles and quads of the other, several result blocks, fewer columns on
+    either side; less than a stage of rows, whole stages and a rest; NaN in
+    columns next to the ones that are read."""
+    rng = np.random.default_rng(1000 * m + k + n)
+    V, W = rng.standard_normal((n, m + 2)), rng.standard_normal((n, k + 2))
+    V[:, 0] = V[:, -1] = W[:, 0] = W[:, -1] = np.nan
+    dV, dW = DeviceMultiVec.from_host(V), DeviceMultiVec.from_host(W)
+    print(f"Gram n={n} m={m} k={k}", flush=True)
+    G = np.zeros((m, k), order="F")
+    _native.hip().GCGE_HIP_Gram(dV.handle, 1, m, dW.handle, 1, k, _native.as_dptr(G), m)
+    V, W = V[:, 1:-1], W[:, 1:-1]
+    assert np.all(np.abs(G - V.T @ W) <= 2 * (n + 2) * EPS * (np.abs(V).T @ np.abs(W)))
