@@ -112,7 +112,8 @@ class DeviceMatrix:
     def set_storage(self, storage) -> bool:
         """Products through "diagonal" storage (when the matrix has it),
         "sliced" ELLPACK with element gathers, or sliced ELLPACK with "rows"
-        gathers from a row-major copy of the column block (from 16 columns);
+        gathers from a row-major copy of the column block (from 8
+        columns, 12 below 65536 rows);
         True/False mean "diagonal"/"sliced".  "diagonal-consecutive" and
         "diagonal-planes" fix the order of the diagonal row blocks,
         "diagonal-tiles" uses the LDS plane tiles of 27-point plane layouts

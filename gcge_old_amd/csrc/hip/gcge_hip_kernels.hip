@@ -856,7 +856,17 @@ __global__ __launch_bounds__(kBlock) void k_cols_to_rows(int n, int k, const T *
     }
 }
 
-template <typename VT, typename XT, int DOT>
+// CPL consecutive columns per lane (64 CPL columns per pass, grid y the
+// passes): one 16-byte load per lane and entry from 65 float64 or 129 float32
+// columns.  Lanes past the last column repeat it, so that the sixteen gathers
+// of an entry row go out together, without branches around them (a predicate
+// on the gathers serialised them behind their index loads); column indices
+// and values are wave-uniform (scalar loads), the indices one entry row ahead.
+// Bound by the random rows of XT from HBM (4.5 TB/s of gathered bytes) at
+// wide blocks.  Measured on the permuted 128^3 K (with the copy): 100 columns
+// 11.1 -> 8.5 ms, 64 4.8 ms, 20 6.0 -> 2.2, permuted 64^3 K: 70 columns 802 ->
+// 537 us, 16 525 -> 192.
+template <typename VT, typename XT, int CPL, int DOT>
 __global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, int slices_per_block,
                                                           const int *__restrict__ sptr,
                                                           const int *__restrict__ sw,
@@ -868,135 +878,95 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, i
                                                           double *__restrict__ dpart, int nparts,
                                                           const int *__restrict__ count)
 {
-    __shared__ double red[DOT > 0 ? 2 * kBlock : 1];
-    const int wid = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    typedef XT Vec __attribute__((ext_vector_type(CPL)));
+    __shared__ double red[DOT > 0 ? 2 * CPL * kBlock : 1];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const int kc = count ? min(k, *count) : k;
-    const int c0 = blockIdx.y * kWave;
+    const int c0 = blockIdx.y * kWave * CPL;
     if (c0 >= kc) return;  // the whole workgroup: same column pass
-    const int c = c0 + lane;
-    const bool live = c < kc;
-    const int s0 = blockIdx.x * slices_per_block, s1 = min(nslices, s0 + slices_per_block);
-    double pw = 0.0, pp = 0.0;
+    const int c = c0 + CPL * lane;
+    // kp is a multiple of CPL: the last group of columns lies inside a row
+    const XT *xl = XTm + min(c, (kc - 1) / CPL * CPL);
+    auto gather = [&](int col) { return *reinterpret_cast<const Vec *>(xl + (long)col * kp); };
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    const int s0 = blk * slices_per_block, s1 = min(nslices, s0 + slices_per_block);
+    double pw[CPL] = {}, pp[CPL] = {};
     for (int sl = s0; sl < s1; ++sl) {
         const int w = sw[sl];
-        const int base = sptr[sl] + wid * kRowsPerWave;
-        XT acc[kRowsPerWave];
+        const int *cp = scol + sptr[sl] + wid * kRowsPerWave;
+        const VT *vp = sval + sptr[sl] + wid * kRowsPerWave;
+        Vec acc[kRowsPerWave] = {};
+        int col[kRowsPerWave];
+        if (w > 0) {
 #pragma unroll
-        for (int i = 0; i < kRowsPerWave; ++i) acc[i] = XT(0);
+            for (int i = 0; i < kRowsPerWave; ++i) col[i] = cp[i];
+        }
         for (int j = 0; j < w; ++j) {
-            const int e0 = base + j * kWave;
-            XT xv[kRowsPerWave];
+            Vec xv[kRowsPerWave];
+#pragma unroll
+            for (int i = 0; i < kRowsPerWave; ++i) xv[i] = gather(col[i]);
+            const int *cn = cp + (long)min(j + 1, w - 1) * kWave;
+            XT v[kRowsPerWave];
 #pragma unroll
             for (int i = 0; i < kRowsPerWave; ++i) {
-                const int col = scol[e0 + i];
-                xv[i] = live ? XTm[(long)col * kp + c] : XT(0);
+                col[i] = cn[i];
+                v[i] = (XT)vp[(long)j * kWave + i];
             }
+            __builtin_amdgcn_sched_barrier(0);  // all in flight before the first use
 #pragma unroll
-            for (int i = 0; i < kRowsPerWave; ++i) acc[i] += (XT)sval[e0 + i] * xv[i];
+            for (int i = 0; i < kRowsPerWave; ++i) {
+#pragma unroll
+                for (int u = 0; u < CPL; ++u) acc[i][u] += v[i] * xv[i][u];
+            }
         }
         const int rbase = sl * kWave + wid * kRowsPerWave;
-        if (live) {
-            XT *y = Y + (long)(ymap ? ymap[c] : c) * ldy;
+#pragma unroll
+        for (int u = 0; u < CPL; ++u) {
+            if (c + u >= kc) continue;
+            XT *y = Y + (long)(ymap ? ymap[c + u] : c + u) * ldy;
 #pragma unroll
             for (int i = 0; i < kRowsPerWave; ++i)
-                if (rbase + i < n) y[rbase + i] = acc[i];
+                if (rbase + i < n) y[rbase + i] = acc[i][u];
         }
         if constexpr (DOT > 0) {
 #pragma unroll
             for (int i = 0; i < kRowsPerWave; ++i) {
                 const int r = rbase + i;
-                const double pv = (live && r < n) ? (double)XTm[(long)r * kp + c] : 0.0;
-                pw += pv * (double)acc[i];
-                if constexpr (DOT > 1) pp += pv * pv;
+                if (r >= n) continue;
+                const Vec p = gather(r);
+#pragma unroll
+                for (int u = 0; u < CPL; ++u) {
+                    pw[u] += (double)p[u] * (double)acc[i][u];
+                    if constexpr (DOT > 1) pp[u] += (double)p[u] * (double)p[u];
+                }
             }
         }
     }
     if constexpr (DOT > 0) {
-        red[threadIdx.x] = pw;
-        red[kBlock + threadIdx.x] = pp;
+#pragma unroll
+        for (int u = 0; u < CPL; ++u) {
+            red[u * kBlock + threadIdx.x] = pw[u];
+            red[(CPL + u) * kBlock + threadIdx.x] = pp[u];
+        }
         __syncthreads();
-        if (wid == 0 && live) {
+        if (wid > 0) return;
+#pragma unroll
+        for (int u = 0; u < CPL; ++u) {
+            if (c + u >= kc) continue;
             double a = 0.0, b = 0.0;
             for (int q = 0; q < kBlock / kWave; ++q) {
-                a += red[q * kWave + lane];
-                b += red[kBlock + q * kWave + lane];
+                a += red[u * kBlock + q * kWave + lane];
+                b += red[(CPL + u) * kBlock + q * kWave + lane];
             }
-            dpart[(long)c * nparts + blockIdx.x] = a;
-            if constexpr (DOT > 1) dpart[(long)(k + c) * nparts + blockIdx.x] = b;
+            dpart[(long)(c + u) * nparts + blk] = a;
+            if constexpr (DOT > 1) dpart[(long)(k + c + u) * nparts + blk] = b;
         }
     }
 }
 
-// The same product with the column passes of a row group in one workgroup:
-// wave w takes columns 64 w .. 64 w + 63 (k <= 256) of every row group of the
-// workgroup's slices, so the four 512-byte pieces of a gathered row of XT
-// are read by the four waves close together in time, instead of by
-// workgroups of different passes far apart.  Each row is summed as in
-// k_sell_rows_spmm; the p.w partial of a column comes from the one wave that
-// owns it.
-template <typename VT, typename XT, int DOT>
-__global__ __launch_bounds__(kBlock) void k_sell_rows_spmm_passes(
-    int n, int nslices, int slices_per_block, const int *__restrict__ sptr,
-    const int *__restrict__ sw, const int *__restrict__ scol, const VT *__restrict__ sval,
-    const XT *__restrict__ XTm, int kp, XT *__restrict__ Y, long ldy, int k,
-    const int *__restrict__ ymap, double *__restrict__ dpart, int nparts,
-    const int *__restrict__ count)
-{
-    const int wid = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int kc = count ? min(k, *count) : k;
-    const int c0 = wid * kWave;
-    if (c0 >= kc) return;  // the whole wave: one column pass
-    const int c = c0 + lane;
-    const bool live = c < kc;
-    XT *y = live ? Y + (long)(ymap ? ymap[c] : c) * ldy : nullptr;
-    const int s0 = blockIdx.x * slices_per_block, s1 = min(nslices, s0 + slices_per_block);
-    double pw = 0.0, pp = 0.0;
-    for (int sl = s0; sl < s1; ++sl) {
-        const int w = sw[sl];
-        for (int g = 0; g < kWave / kRowsPerWave; ++g) {
-            const int base = sptr[sl] + g * kRowsPerWave;
-            XT acc[kRowsPerWave];
-#pragma unroll
-            for (int i = 0; i < kRowsPerWave; ++i) acc[i] = XT(0);
-            for (int j = 0; j < w; ++j) {
-                const int e0 = base + j * kWave;
-                XT xv[kRowsPerWave];
-#pragma unroll
-                for (int i = 0; i < kRowsPerWave; ++i) {
-                    const int col = scol[e0 + i];
-                    xv[i] = live ? XTm[(long)col * kp + c] : XT(0);
-                }
-#pragma unroll
-                for (int i = 0; i < kRowsPerWave; ++i) acc[i] += (XT)sval[e0 + i] * xv[i];
-            }
-            const int rbase = sl * kWave + g * kRowsPerWave;
-            if (live) {
-#pragma unroll
-                for (int i = 0; i < kRowsPerWave; ++i)
-                    if (rbase + i < n) y[rbase + i] = acc[i];
-            }
-            if constexpr (DOT > 0) {
-#pragma unroll
-                for (int i = 0; i < kRowsPerWave; ++i) {
-                    const int r = rbase + i;
-                    const double pv = (live && r < n) ? (double)XTm[(long)r * kp + c] : 0.0;
-                    pw += pv * (double)acc[i];
-                    if constexpr (DOT > 1) pp += pv * pv;
-                }
-            }
-        }
-    }
-    if constexpr (DOT > 0) {
-        if (live) {
-            dpart[(long)c * nparts + blockIdx.x] = pw;
-            if constexpr (DOT > 1) dpart[(long)(k + c) * nparts + blockIdx.x] = pp;
-        }
-    }
-}
-
-// slices per workgroup of the row-gather product: about 2048 workgroups per
+// slices per workgroup of the row-gather product: about 8192 workgroups per
 // column pass
-inline int rows_slices_per_block(const Mat *A) { return std::max(1, (A->nslices + 2047) / 2048); }
+inline int rows_slices_per_block(const Mat *A) { return std::max(1, (A->nslices + 8191) / 8192); }
 inline int rows_parts(const Mat *A)
 {
     const int spb = rows_slices_per_block(A);
@@ -1015,26 +985,27 @@ void launch_rows_spmm(const Mat *A, const VT *vals, const XT *X, long ldx, XT *Y
                        state().stream, A->ncols, k, X, ldx, d_xmap, XTm, kp, d_count);
     const int spb = rows_slices_per_block(A);
     const int nparts = rows_parts(A);
-    static const int passes_mode = [] {
-        const char *e = getenv("GCGE_HIP_ROWS_PASSES");  // "0": one pass per workgroup (measurement)
-        return e ? atoi(e) : 1;
-    }();
-    const int npass = (k + kWave - 1) / kWave;
-    if (passes_mode != 0 && npass >= 2 && npass <= kBlock / kWave)
-        hipExtLaunchKernelGGL((k_sell_rows_spmm_passes<VT, XT, DOT>), dim3(nparts), dim3(kBlock), 0,
-                              state().stream, ev0, ev1, 0, n, A->nslices, spb, A->d_slice_ptr,
-                              A->d_slice_w, A->d_col, vals, XTm, kp, Y, ldy, k, d_ymap, dpart,
-                              nparts, d_count);
-    else
-        hipExtLaunchKernelGGL((k_sell_rows_spmm<VT, XT, DOT>), dim3(nparts, npass), dim3(kBlock), 0,
-                              state().stream, ev0, ev1, 0, n, A->nslices, spb, A->d_slice_ptr,
-                              A->d_slice_w, A->d_col, vals, XTm, kp, Y, ldy, k, d_ymap, dpart,
-                              nparts, d_count);
+#define GCGE_ROWS(CPL)                                                                                   \
+    hipExtLaunchKernelGGL((k_sell_rows_spmm<VT, XT, CPL, DOT>),                                          \
+                          dim3(nparts, (k + CPL * kWave - 1) / (CPL * kWave)), dim3(kBlock), 0,          \
+                          state().stream, ev0, ev1, 0, n, A->nslices, spb, A->d_slice_ptr, A->d_slice_w, \
+                          A->d_col, vals, XTm, kp, Y, ldy, k, d_ymap, dpart, nparts, d_count)
+    if (k <= kWave) {
+        GCGE_ROWS(1);
+    } else if (sizeof(XT) == 8 || k <= 2 * kWave) {
+        GCGE_ROWS(2);
+    } else if constexpr (sizeof(XT) == 4) {
+        GCGE_ROWS(4);
+    }
+#undef GCGE_ROWS
     HIP_CHECK(hipGetLastError());
 }
 
-// the row-gather form from this many columns (fewer leave most lanes idle)
-constexpr int kRowsMinCols = 16;
+// the row-gather form from this many columns (permuted matrices, element
+// against row gathers with their copy: 128^3 K, 8 columns 5508 against 1412
+// us; 64^3 K, 8 columns 321 against 185, 4 columns 125 against 187; 30^3 M, 8
+// columns 31.4 against 34.5, 16 columns 44.8 against 38.8)
+inline int rows_min_cols(const Mat *A) { return A->nrows >= 65536 ? 8 : 12; }
 
 __global__ __launch_bounds__(kBlock) void k_to_float(size_t len, const double *__restrict__ src,
                                                     float *__restrict__ dst)
@@ -2254,7 +2225,7 @@ void spmm(const Mat *A, const double *X, long ldx, double *Y, long ldy, int k, c
     else if (A->use_dia)
         launch_dia_spmm<0>(A, A->d_dia, X, ldx, Y, ldy, k, d_xmap, d_ymap, nullptr, nullptr,
                            prof.start_event(), prof.stop_event());
-    else if (A->use_rows && k >= kRowsMinCols)
+    else if (A->use_rows && k >= rows_min_cols(A))
         launch_rows_spmm<0>(A, A->d_val, X, ldx, Y, ldy, k, d_xmap, d_ymap, nullptr, nullptr,
                             prof.start_event(), prof.stop_event());
     else
@@ -2276,7 +2247,7 @@ void spmm(const Mat *A, const float *X, long ldx, float *Y, long ldy, int k, con
     else if (A->use_dia && A->d_dia32)
         launch_dia_spmm<0>(A, A->d_dia32, X, ldx, Y, ldy, k, d_xmap, d_ymap, nullptr, nullptr,
                            prof.start_event(), prof.stop_event());
-    else if (A->use_rows && k >= kRowsMinCols)
+    else if (A->use_rows && k >= rows_min_cols(A))
         launch_rows_spmm<0>(A, A->d_val32, X, ldx, Y, ldy, k, d_xmap, d_ymap, nullptr, nullptr,
                             prof.start_event(), prof.stop_event());
     else
@@ -2292,7 +2263,7 @@ void spmm_dot(const Mat *A, const double *P, long ldp, double *W, long ldw, int 
     // P read and W written (the p.w epilogue reuses the P values the product reads)
     const double bytes = (double)A->nnz * (8 + 4) + 4.0 * (A->nrows + 1) +
                          8.0 * (double)k * ((double)A->ncols + A->nrows);
-    const bool rows = !A->use_dia && A->use_rows && k >= kRowsMinCols;
+    const bool rows = !A->use_dia && A->use_rows && k >= rows_min_cols(A);
     const bool tiles = A->use_dia && use_tiles<double>(A, k);
     const int nparts = tiles ? tile_parts<double>(A)
                              : (A->use_dia ? dia_blocks(A) : (rows ? rows_parts(A) : A->nslices));
@@ -2326,7 +2297,7 @@ void spmm_dot(const Mat *A, const float *P, long ldp, float *W, long ldw, int k,
     const double bytes = (double)A->nnz * (4 + 4) + 4.0 * (A->nrows + 1) +
                          4.0 * (double)k * ((double)A->ncols + A->nrows);
     const bool dia = A->use_dia && A->d_dia32;
-    const bool rows = !dia && A->use_rows && k >= kRowsMinCols;
+    const bool rows = !dia && A->use_rows && k >= rows_min_cols(A);
     const bool tiles = dia && use_tiles<float>(A, k);
     const int nparts = tiles ? tile_parts<float>(A)
                              : (dia ? dia_blocks(A) : (rows ? rows_parts(A) : A->nslices));

@@ -5,7 +5,7 @@ roundings an entry passes through times the sum of its absolute products."""
 import numpy as np
 import pytest
 
-from gcge_old_amd import DeviceMultiVec, _native, adjoint
+from gcge_old_amd import DeviceMatrix, DeviceMultiVec, _native, adjoint, problems
 from oracle import adjoint as oadj
 
 pytestmark = pytest.mark.gpu
@@ -103,3 +103,47 @@ def test_gram_tiles(n, m, k):
     _native.hip().GCGE_HIP_Gram(dV.handle, 1, m, dW.handle, 1, k, _native.as_dptr(G), m)
     V, W = V[:, 1:-1], W[:, 1:-1]
     assert np.all(np.abs(G - V.T @ W) <= 2 * (n + 2) * EPS * (np.abs(V).T @ np.abs(W)))
+
+
+def _permuted_q1(E, seed):
+    K = problems.q1_fem_3d(E, problems.lognormal_kappa(E, seed))[0]
+    return problems.symmetric_permutation(K, np.random.default_rng(seed).permutation(K.nrows))
+
+
+@pytest.mark.parametrize("k", [11, 12, 13, 63, 64, 65, 127, 128, 129, 200])
+def test_row_gather_product_widths(k):
+    """Below and from the smallest width of the row gathers, one and two
+    columns per lane, one and two passes, odd last columns; bit for bit the
+    sums of the element gathers (the same order)."""
+    A = DeviceMatrix(_permuted_q1(9, 3))
+    assert A.storage_info()["storage"] == "rows"
+    X = np.random.default_rng(k).standard_normal((A.nrows, k + 1))
+    dX, dY, dZ = DeviceMultiVec.from_host(X), DeviceMultiVec(A.nrows, k + 1), DeviceMultiVec(A.nrows, k)
+    lib = _native.hip()
+    print(f"row gathers k={k}", flush=True)
+    lib.GCGE_HIP_SpMM(A.handle, dX.handle, 1, dY.handle, 0, k)
+    A.set_storage("sliced")
+    lib.GCGE_HIP_SpMM(A.handle, dX.handle, 1, dZ.handle, 0, k)
+    np.testing.assert_array_equal(dY.get(0, k), dZ.get())
+    assert np.all(dY.get(k, 1) == 0.0)
+
+
+@pytest.mark.parametrize("fp32,k,rtol", [(False, 70, 1e-10), (False, 131, 1e-10), (True, 70, 1e-4),
+                                         (True, 131, 1e-4), (True, 20, 1e-4)])
+def test_row_gather_block_cg(fp32, k, rtol):
+    """p.w and p.p of the row gathers (one to four columns per lane, last pass
+    partly filled) inside the block CG, against the element gathers."""
+    A = DeviceMatrix(_permuted_q1(9, 4))
+    rng = np.random.default_rng(k)
+    b, x0 = rng.standard_normal((A.nrows, k)), np.zeros((A.nrows, k))
+    lib = _native.hip()
+    out = []
+    for storage in ("rows", "sliced"):
+        A.set_storage(storage)
+        A.set_precision(fp32)
+        R, X = DeviceMultiVec.from_host(b), DeviceMultiVec.from_host(x0)
+        lib.GCGE_HIP_SetLinearSolverParams(8, 1e-30, 0, 0.0, None)
+        lib.GCGE_HIP_MultiLinearSolve(A.handle, R.handle, 0, X.handle, 0, k)
+        lib.GCGE_HIP_SetLinearSolverParams(20, 1e-2, 0, 0.0, None)
+        out.append(X.get())
+    assert np.linalg.norm(out[0] - out[1]) <= rtol * np.linalg.norm(out[1])
