@@ -2480,10 +2480,17 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
     }
     State &s = state();
     const long mk = (long)m * k;
-    double *d_out = small_buffer2((size_t)mk);
-    gram_impl(n, V, ldv, m, W, ldw, k, d_out, nullptr, 0, true);
     double *h = result_buffer((size_t)mk);
-    HIP_CHECK(hipMemcpyAsync(h, d_out, mk * sizeof(double), hipMemcpyDeviceToHost, s.stream));
+    // results of up to 128 KiB: the reduction writes them to the pinned buffer
+    // itself, without a copy behind it (n = 250 047, whole call: 60 x 10 43.2 ->
+    // 42.2 us, 50 x 50 63.3 -> 54.0, 100 x 100 158 -> 151)
+    if (mk <= 16384 && !use_blas()) {
+        gram_impl(n, V, ldv, m, W, ldw, k, h, nullptr, 0, true);
+    } else {
+        double *d_out = small_buffer2((size_t)mk);
+        gram_impl(n, V, ldv, m, W, ldw, k, d_out, nullptr, 0, true);
+        HIP_CHECK(hipMemcpyAsync(h, d_out, mk * sizeof(double), hipMemcpyDeviceToHost, s.stream));
+    }
     if (!sync_result) return;
     HIP_CHECK(hipStreamSynchronize(s.stream));
     for (int j = 0; j < k; ++j)
