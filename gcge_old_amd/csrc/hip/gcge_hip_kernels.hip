@@ -2375,6 +2375,7 @@ static bool use_blas()
     }();
     return v;
 }
+static bool use_blas(int m, int k) { return m > 16 && k > 16 && use_blas(); }
 static rocblas_handle blas_handle()
 {
     static rocblas_handle h = nullptr;
@@ -2411,7 +2412,7 @@ int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw
     State &s = state();
     const long mk = (long)m * k;
     if (partial && (size_t)mk > partial_cap) return -1;
-    if (!partial && use_blas() && m > 16 && k > 16) {
+    if (!partial && use_blas(m, k)) {
         ProfScope prof(profile ? "gram" : nullptr, 8.0 * (double)n * (m + k));
         const double one = 1.0, zero = 0.0;
         if (rocblas_dgemm(blas_handle(), rocblas_operation_transpose, rocblas_operation_none, m, k, n, &one,
@@ -2484,7 +2485,7 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
     // results of up to 128 KiB: the reduction writes them to the pinned buffer
     // itself, without a copy behind it (n = 250 047, whole call: 60 x 10 43.2 ->
     // 42.2 us, 50 x 50 63.3 -> 54.0, 100 x 100 158 -> 151)
-    if (mk <= 16384 && !use_blas()) {
+    if (mk <= 16384 && !use_blas(m, k)) {
         gram_impl(n, V, ldv, m, W, ldw, k, h, nullptr, 0, true);
     } else {
         double *d_out = small_buffer2((size_t)mk);
@@ -2503,7 +2504,7 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
 // row by row.
 void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &out)
 {
-    if (use_blas()) {
+    if (use_blas(m, k)) {
         out.resize((size_t)m * k);
         for (int j = 0; j < k; ++j)
             for (int i = 0; i < m; ++i) out[(size_t)i * k + j] = C[(size_t)j * ldc + i];
@@ -2537,7 +2538,7 @@ void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, dou
         return;
     }
     ProfScope prof("lincomb", 8.0 * (double)n * (m + k) + (beta == 0.0 ? 0.0 : 8.0 * (double)n * k));
-    if (use_blas()) {
+    if (use_blas(m, k)) {
         // Y = beta Y + V C, C^T stored column-major in d_C (leading dimension k)
         const double one = 1.0;
         if (rocblas_dgemm(blas_handle(), rocblas_operation_none, rocblas_operation_transpose, n, k, m, &one, V,
