@@ -1116,18 +1116,26 @@ __device__ __forceinline__ double mfma_quad(double a, double b, double c)
 // 405; at n = 250 047, 60 x 10 36 -> 26 us (5.4 TB/s), 90 x 50 122 -> 65, 20 x
 // 100 118 -> 42 (the wider block takes the part of V).
 // 16-row groups of a stage, as many as the registers of the loads allow, and
-// workgroups per CU (two within 128 registers)
+// the workgroups of eight waves that a CU holds, for which the grid is made:
+// two within 128 registers a lane.  (The bound of the kernel is in waves per
+// SIMD, of which one workgroup has two.)  97 to 100 columns of W (1, 6, 1) take
+// 172 registers, and a grid of two workgroups per CU ran in two rounds: 100 x
+// 100 at n = 42 875, whole call, 64.0 us against 51.1 with one, at 103 823 83.2
+// against 72.2; one 16-row group a stage fits two and takes 55.5 and 78.3.
 __host__ __device__ constexpr int gram_wide_groups(int mi, int nj, int nq)
 {
     return mi == 2 && mi * (4 * nj + nq) <= 16 ? 4 : mi * (4 * nj + nq) <= 52 ? 2 : 1;
 }
 __host__ __device__ constexpr int gram_wide_blocks(int mi, int nj, int nq)
 {
-    return 2 * mi * (4 * nj + nq) + 8 * gram_wide_groups(mi, nj, nq) * mi + 4 * (nj + nq) <= 96 ? 2 : 1;
+    return mi * (4 * nj + nq) <= 24 &&
+                   2 * mi * (4 * nj + nq) + 8 * gram_wide_groups(mi, nj, nq) * mi + 4 * (nj + nq) <= 96
+               ? 2
+               : 1;
 }
 
-template <int MI, int NJ, int NQ>
-__global__ __launch_bounds__(512, gram_wide_blocks(MI, NJ, NQ)) void k_gram_wide(
+template <int MI, int NJ, int NQ, int BLOCKS>
+__global__ __launch_bounds__(512, BLOCKS) void k_gram_wide(
     int n, const double *__restrict__ V, long ldv, int m,
     const double *__restrict__ W, long ldw, int k, double *__restrict__ partial, int mc, int kc,
     int si, int sj)
@@ -1315,8 +1323,8 @@ void launch_gram_wide_q(const GramShape &g, dim3 grid, int n, const double *V, l
 {
     hipStream_t st = state().stream;
 #define GCGE_GW(NQ)                                                                                       \
-    hipLaunchKernelGGL((k_gram_wide<MI, NJ, NQ>), grid, dim3(512), 0, st, n, V, ldv, m, W, ldw, k, partial, \
-                       g.mc, g.kc, si, sj)
+    hipLaunchKernelGGL((k_gram_wide<MI, NJ, NQ, gram_wide_blocks(MI, NJ, NQ)>), grid, dim3(512), 0, st, n, V, \
+                       ldv, m, W, ldw, k, partial, g.mc, g.kc, si, sj)
     if (g.nq == 0) GCGE_GW(0);
     if constexpr (NJ < 7) {
         if (g.nq == 1) GCGE_GW(1);
