@@ -1115,32 +1115,38 @@ __device__ __forceinline__ double mfma_quad(double a, double b, double c)
 // reaches 72.5), 100 x 100 1324 -> 944, 300 x 16 1882 -> 1141, 50 x 50 622 ->
 // 405; at n = 250 047, 60 x 10 36 -> 26 us (5.4 TB/s), 90 x 50 122 -> 65, 20 x
 // 100 118 -> 42 (the wider block takes the part of V).
-// 16-row groups of a stage, as many as the registers of the loads allow, and
-// the workgroups of eight waves that a CU holds, for which the grid is made:
+// 16-row groups of a stage, as many as the registers of the loads allow.
+// Shapes with few products a row (one tile of W, 2 x 2 tiles) take longer
+// stages, that is longer contiguous pieces of every column, where `longer`
+// says so (gram_wide_shape): 2, 4 and 8 groups at n = 2 048 383, whole call, 16
+// x 64 279, 259 and 246 us, 48 x 16 211, 210 and 203, 12 x 8 111, 84 and 72, 200
+// x 8 745 and 643; at n = 103 823 200 x 8 50.0 and 53.6, 48 x 16 29.0, 30.1 and
+// 33.2.
+__host__ __device__ constexpr int gram_wide_groups(int mi, int nj, int nq, int longer)
+{
+    const int c = mi * (4 * nj + nq);
+    if (longer > 0 && mi == 2 && c <= 16) return 4;
+    if (longer > 0 && mi == 1 && nj == 1) return 4 * longer;
+    return c <= 52 ? 2 : 1;
+}
+// The workgroups of eight waves that a CU holds, for which the grid is made:
 // two within 128 registers a lane.  (The bound of the kernel is in waves per
 // SIMD, of which one workgroup has two.)  97 to 100 columns of W (1, 6, 1) take
 // 172 registers, and a grid of two workgroups per CU ran in two rounds: 100 x
 // 100 at n = 42 875, whole call, 64.0 us against 51.1 with one, at 103 823 83.2
 // against 72.2; one 16-row group a stage fits two and takes 55.5 and 78.3.
-__host__ __device__ constexpr int gram_wide_groups(int mi, int nj, int nq)
+__host__ __device__ constexpr int gram_wide_blocks(int mi, int nj, int nq, int g)
 {
-    return mi == 2 && mi * (4 * nj + nq) <= 16 ? 4 : mi * (4 * nj + nq) <= 52 ? 2 : 1;
-}
-__host__ __device__ constexpr int gram_wide_blocks(int mi, int nj, int nq)
-{
-    return mi * (4 * nj + nq) <= 24 &&
-                   2 * mi * (4 * nj + nq) + 8 * gram_wide_groups(mi, nj, nq) * mi + 4 * (nj + nq) <= 96
-               ? 2
-               : 1;
+    const int c = mi * (4 * nj + nq);
+    return c <= 24 && 2 * c + 8 * g * mi + 4 * (nj + nq) <= 96 ? 2 : 1;
 }
 
-template <int MI, int NJ, int NQ, int BLOCKS>
+template <int MI, int NJ, int NQ, int G, int BLOCKS>
 __global__ __launch_bounds__(512, BLOCKS) void k_gram_wide(
     int n, const double *__restrict__ V, long ldv, int m,
     const double *__restrict__ W, long ldw, int k, double *__restrict__ partial, int mc, int kc,
     int si, int sj)
 {
-    constexpr int G = gram_wide_groups(MI, NJ, NQ);    // 16-row groups of a stage
     constexpr int kHalf = NJ * kWave + NQ * 16;        // pairs of W per eight-row half
     constexpr int kPairs = 2 * G * kHalf;
     constexpr int kLoads = (kPairs + 511) / 512;
@@ -1297,9 +1303,9 @@ static int num_cus()
 // x kc columns, mi tiles of V per wave, nj tiles of W and a quad where up to
 // four columns are left over.
 struct GramShape {
-    int gy, gz, mc, kc, mi, nj, nq;
+    int gy, gz, mc, kc, mi, nj, nq, longer;
 };
-inline GramShape gram_wide_shape(int m, int k)
+inline GramShape gram_wide_shape(int n, int m, int k)
 {
     GramShape g;
     g.gz = (k + 127) / 128;
@@ -1314,29 +1320,46 @@ inline GramShape gram_wide_shape(int m, int k)
     g.gy = (ti + most - 1) / most;
     g.mc = (ti + g.gy - 1) / g.gy * 16;
     g.mi = (g.mc / 16 + 7) / 8;
+    // longer stages for blocks beyond the last-level cache (256 MiB: 200 x 8 at n
+    // = 250 047 with two groups 103 us, four 97), the longest from 2^20 rows, as
+    // a workgroup then has 16 of them (n = 857 375, 13 of them: 48 x 8 83 us with
+    // four groups, 87 with eight)
+    g.longer = 8.0 * n * (m + k) <= 256.0 * (1 << 20) ? 0 : n < 1 << 20 ? 1 : 2;
     return g;
 }
 
-template <int MI, int NJ>
+template <int MI, int NJ, int NQ, int G>
+void launch_gram_wide_g(const GramShape &g, dim3 grid, int n, const double *V, long ldv, int m,
+                        const double *W, long ldw, int k, double *partial, int si, int sj)
+{
+    hipLaunchKernelGGL((k_gram_wide<MI, NJ, NQ, G, gram_wide_blocks(MI, NJ, NQ, G)>), grid, dim3(512), 0,
+                       state().stream, n, V, ldv, m, W, ldw, k, partial, g.mc, g.kc, si, sj);
+}
+
+template <int MI, int NJ, int NQ>
 void launch_gram_wide_q(const GramShape &g, dim3 grid, int n, const double *V, long ldv, int m,
                         const double *W, long ldw, int k, double *partial, int si, int sj)
 {
-    hipStream_t st = state().stream;
-#define GCGE_GW(NQ)                                                                                       \
-    hipLaunchKernelGGL((k_gram_wide<MI, NJ, NQ, gram_wide_blocks(MI, NJ, NQ)>), grid, dim3(512), 0, st, n, V, \
-                       ldv, m, W, ldw, k, partial, g.mc, g.kc, si, sj)
-    if (g.nq == 0) GCGE_GW(0);
-    if constexpr (NJ < 7) {
-        if (g.nq == 1) GCGE_GW(1);
-    }
-#undef GCGE_GW
+    constexpr int G0 = gram_wide_groups(MI, NJ, NQ, 0), G1 = gram_wide_groups(MI, NJ, NQ, 1),
+                  G2 = gram_wide_groups(MI, NJ, NQ, 2);
+    if (g.longer == 0 || G1 == G0)
+        launch_gram_wide_g<MI, NJ, NQ, G0>(g, grid, n, V, ldv, m, W, ldw, k, partial, si, sj);
+    else if (g.longer == 1 || G2 == G1)
+        launch_gram_wide_g<MI, NJ, NQ, G1>(g, grid, n, V, ldv, m, W, ldw, k, partial, si, sj);
+    else
+        launch_gram_wide_g<MI, NJ, NQ, G2>(g, grid, n, V, ldv, m, W, ldw, k, partial, si, sj);
 }
 
 void launch_gram_wide(const GramShape &g, int nbx, int n, const double *V, long ldv, int m, const double *W,
                       long ldw, int k, double *partial, int si, int sj)
 {
     const dim3 grid(nbx, g.gy, g.gz);
-#define GCGE_GW_MI(MI, NJ) launch_gram_wide_q<MI, NJ>(g, grid, n, V, ldv, m, W, ldw, k, partial, si, sj)
+#define GCGE_GW_Q(MI, NJ, NQ) launch_gram_wide_q<MI, NJ, NQ>(g, grid, n, V, ldv, m, W, ldw, k, partial, si, sj)
+#define GCGE_GW_MI(MI, NJ)                    \
+    do {                                      \
+        if (g.nq == 0) GCGE_GW_Q(MI, NJ, 0);  \
+        else if constexpr (NJ < 7) GCGE_GW_Q(MI, NJ, 1); \
+    } while (0)
 #define GCGE_GW(NJ)                          \
     case NJ:                                 \
         if (g.mi == 1) GCGE_GW_MI(1, NJ);    \
@@ -1355,6 +1378,7 @@ void launch_gram_wide(const GramShape &g, int nbx, int n, const double *V, long 
     }
 #undef GCGE_GW
 #undef GCGE_GW_MI
+#undef GCGE_GW_Q
     HIP_CHECK(hipGetLastError());
 }
 
@@ -2471,12 +2495,32 @@ int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw
     const double *A = swap ? W : V, *B = swap ? V : W;
     const long lda = swap ? ldw : ldv, ldb = swap ? ldv : ldw;
     const int ma = swap ? k : m, kb = swap ? m : k;
-    const GramShape g = gram_wide_shape(ma, kb);
-    // the workgroups the CUs hold, at least two stages each (at n = 12 167, 50 x
-    // 50: 10.5 us against 12.5 with one, 13.3 with four)
-    const int stage = 16 * gram_wide_groups(g.mi, g.nj, g.nq);
-    const int want = std::max(1, num_cus() * gram_wide_blocks(g.mi, g.nj, g.nq) / (g.gy * g.gz));
-    nbx = gram_ranges(n, std::min(ceil_div(n, 2 * stage), want), mk, partial_cap, 1, &rows);
+    GramShape g = gram_wide_shape(n, ma, kb);
+    // The workgroups the CUs hold, at least two stages each (at n = 12 167, 50 x
+    // 50: 10.5 us against 12.5 with one, 13.3 with four); one per CU where that
+    // leaves the busiest CU at least a ninth fewer rows (whole calls: 256 x 8 at n =
+    // 42 875 44.4 -> 37.3 us with it, 128 x 16 at 17 576 27.9 -> 26.2), or where the
+    // waves have two tiles each and the partials of two would exceed a tenth of
+    // the blocks (256 x 32 at n = 103 823: 77.1 -> 66.3; with one tile a wave 48 x
+    // 48 there takes 35.2 with two and 37.5 with one).
+    const int cus = num_cus(), yz = g.gy * g.gz;
+    auto plan = [&](int longer, int &want) {
+        const int G = gram_wide_groups(g.mi, g.nj, g.nq, longer), stages = ceil_div(n, 16 * G);
+        auto load = [&](int w) { return 16L * G * ceil_div(w * yz, cus) * ceil_div(stages, w); };
+        const int most = ceil_div(stages, 2), one = std::min(most, std::max(1, cus / yz));
+        want = std::min(most, std::max(1, cus * gram_wide_blocks(g.mi, g.nj, g.nq, G) / yz));
+        if (9 * load(one) <= 8 * load(want) || (g.mi > 1 && 10.0 * want * mk > (double)n * (m + k))) want = one;
+        return load(want);
+    };
+    int want = 0, other = 0;
+    const long rows_most = plan(g.longer, want);
+    // two tiles a wave: the longer stage also where the busiest CU has no more
+    // rows with it (n = 27 000, 256 x 8: 32.4 us against 34.1)
+    if (g.longer == 0 && g.mi == 2 && plan(1, other) <= rows_most) {
+        g.longer = 1;
+        want = other;
+    }
+    nbx = gram_ranges(n, want, mk, partial_cap, 1, &rows);
     if (!partial) partial = partial_buffer((size_t)nbx * mk);
     {
         ProfScope prof(pname, gbytes);

@@ -147,3 +147,17 @@ def test_row_gather_block_cg(fp32, k, rtol):
         lib.GCGE_HIP_SetLinearSolverParams(20, 1e-2, 0, 0.0, None)
         out.append(X.get())
     assert np.linalg.norm(out[0] - out[1]) <= rtol * np.linalg.norm(out[1])
+
+
+@pytest.mark.parametrize("n,m,k", [(1100007, 12, 20), (1060003, 17, 16), (600011, 50, 10), (240007, 140, 8),
+                                   (200003, 140, 30), (27001, 200, 8), (17577, 128, 16), (42877, 256, 32)])
+def test_gram_stage_lengths(n, m, k):
+    """Stages of four and eight 16-row groups (blocks beyond 256 MiB, two tiles
+    a wave on a small mesh) with a rest of rows, and one workgroup per CU."""
+    rng = np.random.default_rng(n + m)
+    V, W = rng.standard_normal((n, m)), rng.standard_normal((n, k))
+    dV, dW = DeviceMultiVec.from_host(V), DeviceMultiVec.from_host(W)
+    print(f"Gram n={n} m={m} k={k}", flush=True)
+    G = np.zeros((m, k), order="F")
+    _native.hip().GCGE_HIP_Gram(dV.handle, 0, m, dW.handle, 0, k, _native.as_dptr(G), m)
+    assert np.all(np.abs(G - V.T @ W) <= 2 * (n + 2) * EPS * (np.abs(V).T @ np.abs(W)))
