@@ -113,7 +113,7 @@ class DeviceMatrix:
         """Products through "diagonal" storage (when the matrix has it),
         "sliced" ELLPACK with element gathers, or sliced ELLPACK with "rows"
         gathers from a row-major copy of the column block (from 8
-        columns, 12 below 65536 rows);
+        columns; 12 below 65536 rows, 13 below 12288, 16 below 8192);
         True/False mean "diagonal"/"sliced".  "diagonal-consecutive" and
         "diagonal-planes" fix the order of the diagonal row blocks,
         "diagonal-tiles" uses the LDS plane tiles of 27-point plane layouts

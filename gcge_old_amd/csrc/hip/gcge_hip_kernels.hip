@@ -819,18 +819,32 @@ void launch_dia_tile(const Mat *A, const VT *vals, const XT *X, long ldx, XT *Y,
     HIP_CHECK(hipGetLastError());
 }
 
+// compute units of the device
+static int num_cus()
+{
+    State &s = state();
+    if (!s.cus) {
+        int v = 0;
+        HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, s.device));
+        s.cus = std::max(1, v);
+    }
+    return s.cus;
+}
+
 // ---- SpMM with whole-row gathers (matrices with scattered columns) ------------------
 // The column block X (column-major, optional column map) is first copied to a
 // row-major block XT (row i: the k values of row i, row stride kp), through
 // 64 x 64 LDS tiles so that both sides are coalesced.  The product then runs
 // with lanes along the columns: a wavefront owns 16 rows of a sliced-ELLPACK
-// slice and 64 columns (grid y: column passes); for every entry of those rows
-// the column index and value are wave-uniform, and the gather of the matching
-// row of XT is one contiguous access of 64 values, where the column-major form
-// takes a separate cache line per element.  Each lane writes its 16 outputs
-// of a column as one contiguous run.  DOT: p.w (and p.p) per column, summed
-// over the workgroup's rows through LDS, one partial per workgroup.
+// slice and 64, 128 or 256 columns, one, two or four per lane (grid y: column
+// passes); for every entry of those rows the column index and value are
+// wave-uniform, and the gather of the matching row of XT is one contiguous
+// access, where the column-major form takes a separate cache line per element.
+// Each lane writes its 16 outputs of a column as one contiguous run.  DOT: p.w
+// (and p.p) per column, summed over the workgroup's rows (through LDS where it
+// has several waves), one partial per workgroup.
 constexpr int kRowsPerWave = 16;
+constexpr int kRowGroups = kWave / kRowsPerWave;  // waves of a slice
 
 // (only the first min(k, *count) columns: entries of a device column list
 // beyond its length are not defined)
@@ -866,8 +880,8 @@ __global__ __launch_bounds__(kBlock) void k_cols_to_rows(int n, int k, const T *
 // wide blocks.  Measured on the permuted 128^3 K (with the copy): 100 columns
 // 11.1 -> 8.5 ms, 64 4.8 ms, 20 6.0 -> 2.2, permuted 64^3 K: 70 columns 802 ->
 // 537 us, 16 525 -> 192.
-template <typename VT, typename XT, int CPL, int DOT>
-__global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, int slices_per_block,
+template <typename VT, typename XT, int CPL, int DOT, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void k_sell_rows_spmm(int n, int nslices, int slices_per_block,
                                                           const int *__restrict__ sptr,
                                                           const int *__restrict__ sw,
                                                           const int *__restrict__ scol,
@@ -879,8 +893,9 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, i
                                                           const int *__restrict__ count)
 {
     typedef XT Vec __attribute__((ext_vector_type(CPL)));
-    __shared__ double red[DOT > 0 ? 2 * CPL * kBlock : 1];
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    __shared__ double red[DOT > 0 && WAVES > 1 ? 2 * CPL * kBlock : 1];
+    const int blk = xcd_remap(blockIdx.x, gridDim.x), lane = threadIdx.x % kWave;
+    const int wid = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : blk % kRowGroups;
     const int kc = count ? min(k, *count) : k;
     const int c0 = blockIdx.y * kWave * CPL;
     if (c0 >= kc) return;  // the whole workgroup: same column pass
@@ -888,8 +903,8 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, i
     // kp is a multiple of CPL: the last group of columns lies inside a row
     const XT *xl = XTm + min(c, (kc - 1) / CPL * CPL);
     auto gather = [&](int col) { return *reinterpret_cast<const Vec *>(xl + (long)col * kp); };
-    const int blk = xcd_remap(blockIdx.x, gridDim.x);
-    const int s0 = blk * slices_per_block, s1 = min(nslices, s0 + slices_per_block);
+    const int s0 = WAVES > 1 ? blk * slices_per_block : blk / kRowGroups;
+    const int s1 = WAVES > 1 ? min(nslices, s0 + slices_per_block) : s0 + 1;
     double pw[CPL] = {}, pp[CPL] = {};
     for (int sl = s0; sl < s1; ++sl) {
         const int w = sw[sl];
@@ -942,7 +957,14 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, i
             }
         }
     }
-    if constexpr (DOT > 0) {
+    if constexpr (DOT > 0 && WAVES == 1) {
+#pragma unroll
+        for (int u = 0; u < CPL; ++u) {
+            if (c + u >= kc) continue;
+            dpart[(long)(c + u) * nparts + blk] = pw[u];
+            if constexpr (DOT > 1) dpart[(long)(k + c + u) * nparts + blk] = pp[u];
+        }
+    } else if constexpr (DOT > 0) {
 #pragma unroll
         for (int u = 0; u < CPL; ++u) {
             red[u * kBlock + threadIdx.x] = pw[u];
@@ -967,8 +989,14 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows_spmm(int n, int nslices, i
 // slices per workgroup of the row-gather product: about 8192 workgroups per
 // column pass
 inline int rows_slices_per_block(const Mat *A) { return std::max(1, (A->nslices + 8191) / 8192); }
+// workgroups of one wave up to two slices per CU: the gathers keep the address
+// unit of a CU busy, and a few workgroups of four waves load some CUs with two
+// of them and others with one (permuted K, 13 columns: n = 17 576 28.5 -> 21.4
+// us, 27 000 30.8 -> 28.4; beyond, 64 columns at 42 875 66 against 69)
+inline bool rows_one_wave(const Mat *A) { return A->nslices <= 2 * num_cus(); }
 inline int rows_parts(const Mat *A)
 {
+    if (rows_one_wave(A)) return A->nslices * kRowGroups;
     const int spb = rows_slices_per_block(A);
     return (A->nslices + spb - 1) / spb;
 }
@@ -985,11 +1013,16 @@ void launch_rows_spmm(const Mat *A, const VT *vals, const XT *X, long ldx, XT *Y
                        state().stream, A->ncols, k, X, ldx, d_xmap, XTm, kp, d_count);
     const int spb = rows_slices_per_block(A);
     const int nparts = rows_parts(A);
-#define GCGE_ROWS(CPL)                                                                                   \
-    hipExtLaunchKernelGGL((k_sell_rows_spmm<VT, XT, CPL, DOT>),                                          \
-                          dim3(nparts, (k + CPL * kWave - 1) / (CPL * kWave)), dim3(kBlock), 0,          \
+#define GCGE_ROWS_W(CPL, WAVES)                                                                          \
+    hipExtLaunchKernelGGL((k_sell_rows_spmm<VT, XT, CPL, DOT, WAVES>),                                   \
+                          dim3(nparts, (k + CPL * kWave - 1) / (CPL * kWave)), dim3(WAVES * kWave), 0,   \
                           state().stream, ev0, ev1, 0, n, A->nslices, spb, A->d_slice_ptr, A->d_slice_w, \
                           A->d_col, vals, XTm, kp, Y, ldy, k, d_ymap, dpart, nparts, d_count)
+#define GCGE_ROWS(CPL)                              \
+    do {                                            \
+        if (rows_one_wave(A)) GCGE_ROWS_W(CPL, 1);  \
+        else GCGE_ROWS_W(CPL, kRowGroups);          \
+    } while (0)
     if (k <= kWave) {
         GCGE_ROWS(1);
     } else if (sizeof(XT) == 8 || k <= 2 * kWave) {
@@ -998,14 +1031,26 @@ void launch_rows_spmm(const Mat *A, const VT *vals, const XT *X, long ldx, XT *Y
         GCGE_ROWS(4);
     }
 #undef GCGE_ROWS
+#undef GCGE_ROWS_W
     HIP_CHECK(hipGetLastError());
 }
 
 // the row-gather form from this many columns (permuted matrices, element
-// against row gathers with their copy: 128^3 K, 8 columns 5508 against 1412
-// us; 64^3 K, 8 columns 321 against 185, 4 columns 125 against 187; 30^3 M, 8
-// columns 31.4 against 34.5, 16 columns 44.8 against 38.8)
-inline int rows_min_cols(const Mat *A) { return A->nrows >= 65536 ? 8 : 12; }
+// against row gathers with their copy, us).  From 65536 rows: 64^3 K, 4 columns
+// 125 against 187, 8 columns 321 against 179; at 128^3 8 columns take 5508
+// against 1412, so the forms cross below 8 there; the line keeps to the smaller
+// of these matrices.  Below 65536: at n = 59 319 12 columns of K 67.7 against 50.3
+// (11 by elements 61.3: the line is on the safe side there too), at 27 000 28.7
+// against 28.1, at 17 576 21.8 against 21.3, and fewer columns by elements
+// (17 576: 11 columns 19.9, 27 000: 26.4); at 12 167 12 columns 17.9 against 18.7, 13
+// 19.4 against 18.8; at 9261 13 columns 17.5 against 18.3 of K, 21.9 against 21.2
+// of M; at 6859 15 columns 19.0 against 17.9, 13 15.7 against 17.9; at 3375 16
+// 15.8 against 16.9.
+inline int rows_min_cols(const Mat *A)
+{
+    const int n = A->nrows;
+    return n >= 65536 ? 8 : n >= 12288 ? 12 : n >= 8192 ? 13 : 16;
+}
 
 __global__ __launch_bounds__(kBlock) void k_to_float(size_t len, const double *__restrict__ src,
                                                     float *__restrict__ dst)
@@ -1288,16 +1333,6 @@ __global__ __launch_bounds__(512, BLOCKS) void k_gram_wide(
     }
 }
 
-static int num_cus()
-{
-    State &s = state();
-    if (!s.cus) {
-        int v = 0;
-        HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, s.device));
-        s.cus = std::max(1, v);
-    }
-    return s.cus;
-}
 
 // The result blocks of k_gram_wide for an m x k product: gy x gz blocks of mc
 // x kc columns, mi tiles of V per wave, nj tiles of W and a quad where up to

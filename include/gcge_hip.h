@@ -71,8 +71,8 @@ void GCGE_HIP_MatSetPrecision(void *mat, int fp32);
  * use it.  A matrix most of whose entries sit in sliced-ELLPACK entry rows
  * spanning 256 columns or more (scattered columns, e.g. a random symmetric
  * permutation) instead
- * runs its products of 8 columns or more (12 below 65536 rows) with
- * whole-row gathers from a
+ * runs its products of 8 columns or more (12 below 65536 rows, 13 below
+ * 12288, 16 below 8192) with whole-row gathers from a
  * row-major copy of the column block.  storage: 0 = sliced ELLPACK with
  * element gathers (every matrix has it), 1 = diagonal (when it exists,
  * else 0), 2 = sliced ELLPACK with row gathers.  Returns the storage now

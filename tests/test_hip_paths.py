@@ -161,3 +161,37 @@ def test_gram_stage_lengths(n, m, k):
     G = np.zeros((m, k), order="F")
     _native.hip().GCGE_HIP_Gram(dV.handle, 0, m, dW.handle, 0, k, _native.as_dptr(G), m)
     assert np.all(np.abs(G - V.T @ W) <= 2 * (n + 2) * EPS * (np.abs(V).T @ np.abs(W)))
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("E,k,rows", [(42, 7, False), (42, 8, True), (42, 9, True), (42, 11, True), (32, 12, True),
+                                      (26, 11, False), (26, 12, True), (24, 12, False), (24, 13, True),
+                                      (9, 15, False), (9, 16, True), (9, 129, True), (33, 70, True)])
+def test_row_gather_threshold(E, k, rows, fp32):
+    """Both sides of the smallest width of the row gathers at each size of the
+    rule, one-wave and four-wave workgroups: products bit for bit those of the
+    element gathers; a float64 block CG gives their bits exactly where both
+    storages run them (the forms add p.w up in different orders, which
+    float32 directions round away)."""
+    A = DeviceMatrix(_permuted_q1(E, 5))
+    assert A.storage_info()["storage"] == "rows"
+    rng = np.random.default_rng(100 * E + k)
+    b, x0 = rng.standard_normal((A.nrows, k)), np.zeros((A.nrows, k))
+    lib = _native.hip()
+    print(f"row gathers E={E} k={k} fp32={fp32}", flush=True)
+    out = []
+    for storage in ("rows", "sliced"):
+        A.set_storage(storage)
+        X, Y = DeviceMultiVec.from_host(b), DeviceMultiVec(A.nrows, k)
+        lib.GCGE_HIP_SpMM(A.handle, X.handle, 0, Y.handle, 0, k)
+        A.set_precision(fp32)
+        S = DeviceMultiVec.from_host(x0)
+        lib.GCGE_HIP_SetLinearSolverParams(8, 1e-30, 0, 0.0, None)
+        lib.GCGE_HIP_MultiLinearSolve(A.handle, X.handle, 0, S.handle, 0, k)
+        lib.GCGE_HIP_SetLinearSolverParams(20, 1e-2, 0, 0.0, None)
+        A.set_precision(False)
+        out.append((Y.get(), S.get()))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert np.linalg.norm(out[0][1] - out[1][1]) <= (1e-4 if fp32 else 1e-10) * np.linalg.norm(out[1][1])
+    if not fp32:
+        assert np.array_equal(out[0][1], out[1][1]) == (not rows)
