@@ -1578,6 +1578,92 @@ __global__ __launch_bounds__(kBlock, 4 * NJ + NQ <= 12 ? 4 : 2) void k_lincomb(
     for (int j = 0; j < NQ; ++j) put(16 * NJ + 4 * j + kk, quad[0][j], quad[1][j]);
 }
 
+// Few input columns (lincomb_few): bound by HBM (8 n (m + k) bytes; Y read too
+// for beta != 0), where a wave of k_lincomb has little to do for its rows and
+// k_lincomb_few loads less than the matrix products' whole stages.  A thread
+// owns two rows: its M values of V in registers (columns past m read column m -
+// 1 and count as zero), then every output column of its range, four at a time,
+// as 16-byte accesses; the coefficients (M a column) through LDS.  Whole calls
+// against k_lincomb: n = 2 048 383, 1 -> 1 26.7 -> 12.4 us, 2 -> 2 25.4 -> 16.4, 4 ->
+// 20 109 -> 83, 4 -> 33 230 -> 236; n = 493 039, 8 -> 1 12.7 -> 10.6, 4 -> 4 14.5 ->
+// 12.2; n = 12 167, 3 -> 100 20.0 -> 14.1.
+template <int M>
+__global__ __launch_bounds__(kBlock) void k_lincomb_few(int n, const double *__restrict__ V, long ldv, int m,
+                                                        const double *__restrict__ C, double beta,
+                                                        double *__restrict__ Y, long ldy, int k, int cols)
+{
+    __shared__ double cs[kLcCols * M];
+    const int row = 2 * (blockIdx.x * kBlock + threadIdx.x);
+    const int j0 = blockIdx.y * cols, jn = min(k - j0, cols);
+    // rows past the end repeat the last pair, and are not stored
+    const double *vp = V + min(row, (n - 1) & ~1);
+    gcge_double2 v[M];
+#pragma unroll
+    for (int i = 0; i < M; ++i) v[i] = *reinterpret_cast<const gcge_double2 *>(vp + (long)min(i, m - 1) * ldv);
+    for (int e = threadIdx.x; e < jn * M; e += kBlock) cs[e] = C[(long)j0 * M + e];
+    __syncthreads();
+    if (row >= n) return;
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+        if (i >= m) v[i] = gcge_double2{0.0, 0.0};
+    const bool two = row + 1 < n;
+    double *yp = Y + (long)j0 * ldy + row;
+    for (int j = 0; j < jn; j += 4) {
+        gcge_double2 o[4];
+        if (beta != 0.0) {  // the loads of four columns go out together
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                o[u] = *reinterpret_cast<const gcge_double2 *>(yp + (long)min(j + u, jn - 1) * ldy);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (j + u >= jn) break;
+            const double *c = cs + (j + u) * M;
+            double y0 = 0.0, y1 = 0.0;
+#pragma unroll
+            for (int i = 0; i < M; ++i) {
+                y0 += v[i][0] * c[i];
+                y1 += v[i][1] * c[i];
+            }
+            if (beta != 0.0) {
+                y0 = beta * o[u][0] + y0;
+                y1 = beta * o[u][1] + y1;
+            }
+            double *y = yp + (long)(j + u) * ldy;
+            if (two) *reinterpret_cast<gcge_double2 *>(y) = gcge_double2{y0, y1};
+            else *y = y0;
+        }
+    }
+}
+
+// up to four input columns, up to eight where there are few outputs too (from
+// there on k_lincomb is as quick or quicker: n = 250 047, 8 -> 16 14.1 against 14.9
+// us, n = 2 048 383, 6 -> 16 78 against 82, 7 -> 28 199 against 214)
+inline bool lincomb_few(int m, int k) { return m <= 4 || (m <= 8 && k <= 8); }
+// columns of V that k_lincomb_few is compiled for
+inline int lincomb_few_pad(int m) { return m <= 4 ? m : m <= 6 ? 6 : 8; }
+
+void launch_lincomb_few(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
+                        long ldy, int k, int cols)
+{
+    const dim3 grid((n + 2 * kBlock - 1) / (2 * kBlock), (k + cols - 1) / cols);
+#define GCGE_LC(M)                                                                                           \
+    case M:                                                                                                  \
+        hipLaunchKernelGGL((k_lincomb_few<M>), grid, dim3(kBlock), 0, state().stream, n, V, ldv, m, d_C, beta, \
+                           Y, ldy, k, cols);                                                                 \
+        break
+    switch (lincomb_few_pad(m)) {
+        GCGE_LC(1);
+        GCGE_LC(2);
+        GCGE_LC(3);
+        GCGE_LC(4);
+        GCGE_LC(6);
+        GCGE_LC(8);
+    }
+#undef GCGE_LC
+    HIP_CHECK(hipGetLastError());
+}
+
 // The column groups of a combination with k outputs: `groups` of `cols`
 // columns each (the last may have fewer), as nj tiles of 16 and nq quads.
 struct LcShape {
@@ -2596,14 +2682,23 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
 
 // C (m x k, leading dimension ldc) in the order the combination reads it: per
 // column group, step of 4 input columns, and tile (4 x 16, output column
-// fastest) or quad (4 x 4), zeros past m and k.  For the library comparison:
-// row by row.
+// fastest) or quad (4 x 4), zeros past m and k.  Few input columns: column by
+// column, zeros past m.  For the library comparison: row by row.
 void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &out)
 {
     if (use_blas(m, k)) {
         out.resize((size_t)m * k);
         for (int j = 0; j < k; ++j)
             for (int i = 0; i < m; ++i) out[(size_t)i * k + j] = C[(size_t)j * ldc + i];
+        return;
+    }
+    if (lincomb_few(m, k)) {
+        const int M = lincomb_few_pad(m);
+        // whole 64 bytes: uploads of other sizes take longer (1 -> 33 columns at n =
+        // 12 167 12.2 us a call, with 264 bytes)
+        out.assign(((size_t)k * M + 7) / 8 * 8, 0.0);
+        for (int j = 0; j < k; ++j)
+            for (int i = 0; i < m; ++i) out[(size_t)j * M + i] = C[(size_t)j * ldc + i];
         return;
     }
     const LcShape s = lincomb_shape(k);
@@ -2621,8 +2716,8 @@ void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &o
         }
 }
 
-// the wave that writes a row has read all its inputs, and one group holds
-// every column: the output may overwrite the input
+// the wave (few input columns: the thread) that writes a row has read all its
+// inputs, and one group holds every column: the output may overwrite the input
 bool lincomb_in_place_ok(int m, int k) { return m > 0 && k > 0 && k <= kLcCols && !use_blas(); }
 
 void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
@@ -2644,6 +2739,18 @@ void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, dou
     }
     // multivec columns and scratch blocks start on 512-byte boundaries
     if (!quad_ok(V, ldv) || !quad_ok(Y, ldy)) fail_msg("linear combination: blocks must be 16-byte aligned");
+    if (lincomb_few(m, k)) {
+        // column ranges up to four workgroups per CU, which read V once each: on
+        // small meshes of m or four columns at least, else of 4 m (n = 103 823, 4 ->
+        // 100 23.4 us with five ranges, 25.6 with two).  One range where Y may
+        // overlap V: a thread has read its rows before it writes them.
+        const bool apart = V + (long)(m - 1) * ldv + n <= Y || Y + (long)(k - 1) * ldy + n <= V;
+        const int blocks = ceil_div(n, 2 * kBlock), cus = num_cus();
+        const int least = blocks >= cus ? 4 * m : std::max(4, m);
+        const int parts = apart ? std::max(1, std::min(k / least, 4 * cus / blocks)) : 1;
+        launch_lincomb_few(n, V, ldv, m, d_C, beta, Y, ldy, k, ceil_div(k, std::max(parts, ceil_div(k, kLcCols))));
+        return;
+    }
     launch_lincomb(n, V, ldv, m, d_C, beta, Y, ldy, k);
 }
 

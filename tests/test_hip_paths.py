@@ -195,3 +195,38 @@ def test_row_gather_threshold(E, k, rows, fp32):
     assert np.linalg.norm(out[0][1] - out[1][1]) <= (1e-4 if fp32 else 1e-10) * np.linalg.norm(out[1][1])
     if not fp32:
         assert np.array_equal(out[0][1], out[1][1]) == (not rows)
+
+
+@pytest.mark.parametrize("k", [1, 3, 4, 5, 8, 9, 33, 128, 129, 300])
+@pytest.mark.parametrize("n,m", [(1, 1), (2, 2), (511, 3), (512, 4), (513, 5), (1025, 6), (1003, 7), (2049, 8),
+                                 (140001, 1), (140001, 4)])
+def test_linear_comb_few_inputs(n, m, k):
+    """One to eight input columns (from five on few outputs only), column ranges
+    on both sides of one workgroup per CU, rests of four columns, rows that end
+    inside a pair and a workgroup; infinities stay in their rows; NaN in columns
+    next to the ones that are read; over the input the same bits."""
+    rng = np.random.default_rng(1000 * m + k + n)
+    V = rng.standard_normal((n, m + 2))
+    V[:, 0] = V[:, -1] = np.nan
+    V[n // 2, m] = np.inf
+    C = np.asfortranarray(rng.standard_normal((m, k)))
+    Y0 = rng.standard_normal((n, k + 1))
+    lib = _native.hip()
+    print(f"linear combination n={n} m={m} k={k}", flush=True)
+    rows = np.arange(n) != n // 2
+    for beta in (0.0, -1.5):
+        dV, dY = DeviceMultiVec.from_host(V), DeviceMultiVec.from_host(Y0)
+        lib.GCGE_HIP_LinearComb(dV.handle, 1, m, _native.as_dptr(C), m, beta, dY.handle, 0, k)
+        got = dY.get()
+        want = V[rows, 1:-1] @ C + beta * Y0[rows, :k]
+        bound = np.abs(V[rows, 1:-1]) @ np.abs(C) + abs(beta) * np.abs(Y0[rows, :k])
+        assert np.all(np.abs(got[rows, :k] - want) <= 2 * (m + 2) * EPS * bound)
+        np.testing.assert_array_equal(got[n // 2, :k], np.inf * C[m - 1])
+        np.testing.assert_array_equal(got[:, k:], Y0[:, k:])
+    if k <= 128:
+        A = np.zeros((n, max(m, k) + 1))
+        A[:, :m] = V[:, 1:-1]
+        dA, dY = DeviceMultiVec.from_host(A), DeviceMultiVec(n, k)
+        lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dY.handle, 0, k)
+        lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dA.handle, 1, k)
+        np.testing.assert_array_equal(dA.get(1, k), dY.get())
