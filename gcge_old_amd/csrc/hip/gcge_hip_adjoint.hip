@@ -220,14 +220,15 @@ void q1_element_gradient(int E, const double *X, long ldx, const double *Y, long
     if (E < 2 || k <= 0) return;
     const long ne = (long)E * E * E;
     const double h = 1.0 / E;
-    ProfScope prof("q1_elem_grad", 16.0 * k * (double)(E - 1) * (E - 1) * (E - 1) + 8.0 * ne);
+    const bool same = X == Y && ldx == ldy;  // read once
+    ProfScope prof("q1_elem_grad", (same ? 8.0 : 16.0) * k * (double)(E - 1) * (E - 1) * (E - 1) + 8.0 * ne);
     // eight planes per thread (two operands: four, for the registers) where
     // that gives six wavefronts per CU, from about E = 90: 617 against 712 us
     // at 128^3 x 100, 86 against 91 at 97^3 x 33; below, four planes and the
     // columns of X shared by four threads: 21 against 28 us at 64^3 x 20, 15
     // against 68 at 24^3 x 60
     const long waves = ((long)E * E + kWave - 1) / kWave * ((E + 7) / 8);
-    const bool many = waves >= 6L * 256, same = X == Y && ldx == ldy;
+    const bool many = waves >= 6L * num_cus();
     if (many && same)
         launch_elem_grad<8, 1, true>(E, h / 36.0, X, ldx, Y, ldy, k, d_w, d_node_row, d_grad);
     else if (many)

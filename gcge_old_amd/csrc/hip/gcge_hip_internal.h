@@ -53,6 +53,7 @@ struct State {
 };
 State &state();
 int ensure_init();
+int num_cus();  // compute units of the device
 
 double *partial_buffer(size_t doubles);
 double *small_buffer(size_t doubles);

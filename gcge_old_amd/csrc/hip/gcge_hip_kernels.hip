@@ -33,6 +33,17 @@
 
 namespace gcge_hip {
 
+int num_cus()
+{
+    State &s = state();
+    if (!s.cus) {
+        int v = 0;
+        HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, s.device));
+        s.cus = std::max(1, v);
+    }
+    return s.cus;
+}
+
 namespace {
 
 constexpr int kWave = 64;
@@ -817,18 +828,6 @@ void launch_dia_tile(const Mat *A, const VT *vals, const XT *X, long ldx, XT *Y,
     else GCGE_TILE_LAUNCH(2, 3);
 #undef GCGE_TILE_LAUNCH
     HIP_CHECK(hipGetLastError());
-}
-
-// compute units of the device
-static int num_cus()
-{
-    State &s = state();
-    if (!s.cus) {
-        int v = 0;
-        HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, s.device));
-        s.cus = std::max(1, v);
-    }
-    return s.cus;
 }
 
 // ---- SpMM with whole-row gathers (matrices with scattered columns) ------------------

@@ -2,6 +2,8 @@
 wrong: tile edges, remainders, the smallest sizes and both sides of a rule
 (GPU).  Tolerances are forward-error bounds: unit roundoff times the number of
 roundings an entry passes through times the sum of its absolute products."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -230,3 +232,21 @@ def test_linear_comb_few_inputs(n, m, k):
         lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dY.handle, 0, k)
         lib.GCGE_HIP_LinearComb(dA.handle, 0, m, _native.as_dptr(C), m, 0.0, dA.handle, 1, k)
         np.testing.assert_array_equal(dA.get(1, k), dY.get())
+
+
+@pytest.mark.parametrize("two_blocks", [False, True])
+def test_element_gradient_reported_bytes(two_blocks):
+    """The gradient's recorded traffic: X once where Y is X, else both blocks."""
+    E, k = 20, 7
+    X = DeviceMultiVec.from_host(np.random.default_rng(0).standard_normal(((E - 1) ** 3, k)))
+    Y = DeviceMultiVec.from_host(np.ones(((E - 1) ** 3, k))) if two_blocks else None
+    lib = _native.hip()
+    lib.GCGE_HIP_ProfileReset()
+    lib.GCGE_HIP_ProfileEnable(1)
+    adjoint.q1_kappa_gradient(E, X, np.ones(k), Y=Y)
+    lib.GCGE_HIP_ProfileEnable(0)
+    ms, count, moved = ctypes.c_double(), ctypes.c_int(), ctypes.c_double()
+    lib.GCGE_HIP_KernelStats(b"q1_elem_grad", ctypes.byref(ms), ctypes.byref(count), ctypes.byref(moved))
+    lib.GCGE_HIP_ProfileReset()
+    assert count.value == 1
+    assert moved.value == 8.0 * ((2 if two_blocks else 1) * k * (E - 1) ** 3 + E ** 3)
