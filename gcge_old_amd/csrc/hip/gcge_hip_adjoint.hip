@@ -26,16 +26,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWave = 64;
-constexpr int kXcds = 8;
-
-// Workgroup b is dispatched to XCD b % 8.  Renumber so that the workgroups of
-// one XCD cover one contiguous range of work items.
-__device__ __forceinline__ int xcd_remap(int bid, int nb)
-{
-    const int q = nb / kXcds, r = nb % kXcds;
-    const int xcd = bid % kXcds, loc = bid / kXcds;
-    return (xcd < r) ? xcd * (q + 1) + loc : r * (q + 1) + (xcd - r) * q + loc;
-}
 
 __global__ __launch_bounds__(kBlock) void k_pattern_grad(int n, int nslices,
                                                         const int *__restrict__ sptr,

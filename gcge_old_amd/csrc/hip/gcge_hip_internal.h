@@ -9,6 +9,17 @@
 
 namespace gcge_hip {
 
+constexpr int kXcds = 8;
+
+// Workgroup b is dispatched to XCD b % 8.  Renumber so that the workgroups of
+// one XCD cover one contiguous range of work items.
+__device__ __forceinline__ int xcd_remap(int bid, int nb)
+{
+    const int q = nb / kXcds, r = nb % kXcds;
+    const int xcd = bid % kXcds, loc = bid / kXcds;
+    return (xcd < r) ? xcd * (q + 1) + loc : r * (q + 1) + (xcd - r) * q + loc;
+}
+
 // ---- error handling --------------------------------------------------------
 void fail(const char *what, hipError_t err, const char *file, int line);
 #define HIP_CHECK(expr)                                                       \

@@ -48,16 +48,6 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
-constexpr int kXcds = 8;
-
-// Workgroup b is dispatched to XCD b % 8.  Renumber so that the workgroups of
-// one XCD cover one contiguous range of work items.
-__device__ __forceinline__ int xcd_remap(int bid, int nb)
-{
-    const int q = nb / kXcds, r = nb % kXcds;
-    const int xcd = bid % kXcds, loc = bid / kXcds;
-    return (xcd < r) ? xcd * (q + 1) + loc : r * (q + 1) + (xcd - r) * q + loc;
-}
 
 // DPP move of a double (two 32-bit halves); lanes without a source, or in
 // rows outside ROW_MASK, get 0
@@ -1476,9 +1466,14 @@ __global__ __launch_bounds__(kBlock, 4 * NJ + NQ <= 12 ? 4 : 2) void k_lincomb(
     int n, const double *__restrict__ V, long ldv, int m, const double *__restrict__ Cp, double beta,
     double *__restrict__ Y, long ldy, int k, int group_cols)
 {
-    // four steps where the accumulators fill the registers (three instead of two
-    // waves per SIMD: 200 -> 116 columns 2031 -> 1662 us; 300 -> 64 the other way
-    // round, 1497 against 1573)
+    // four steps where the accumulators fill the registers: with eight, 101 to 104
+    // and 121 to 124 columns need all 256 and spill (eight -> four: 200 -> 116 columns
+    // at n = 2 048 383 2031 -> 1662 us, 60 -> 121 at 250 047 132 -> 122); 300 -> 64 the
+    // other way round, 1497 against 1573.  101 to 108 and 121 to 124 columns (6, 2), (6, 3)
+    // and (7, 3) still run two waves per SIMD (172 registers), and a bound of
+    // three would spill; 41 to 44 columns (2, 3) spill two registers under their
+    // bound of four and are as quick with it as without (300 -> 44 at n = 103 823
+    // 82.8 us against 83.9, 200 -> 44 at 493 039 220.3 against 219.9).
     constexpr int S = NJ >= 5 ? kLcSteps / 2 : kLcSteps;
     constexpr int kStep = NJ * kWave + NQ * 16;  // packed coefficients of a step
     constexpr int kStage2 = S * kStep / 2;  // pairs of a stage
@@ -2554,17 +2549,14 @@ static bool quad_ok(const T *base, long ld)
     return ((uintptr_t)base % 16) == 0 && ((size_t)ld * sizeof(T)) % 16 == 0;
 }
 
-// The row ranges of a Gram launch: as many as `want`, or fewer when the
-// caller's partial buffer (cap doubles, 0: the backend's grown buffer)
-// cannot hold that many m x k blocks; rows per range rounded up to `gran`.
-static int gram_ranges(int n, int want, long mk, size_t cap, int gran, int *rows)
+// The workgroups (and row ranges) of a Gram launch: as many as `want`, or fewer
+// when the caller's partial buffer (cap doubles, 0: the backend's grown buffer)
+// cannot hold that many m x k blocks; no empty ranges of ceil(n / ranges) rows.
+static int gram_ranges(int n, int want, long mk, size_t cap)
 {
     int nbx = std::max(1, want);
     if (cap && (size_t)nbx * mk > cap) nbx = (int)std::max<size_t>(1, cap / mk);
-    int r = ceil_div(n, nbx);
-    r = (r + gran - 1) / gran * gran;
-    *rows = r;
-    return std::max(1, ceil_div(n, r));
+    return std::max(1, ceil_div(n, ceil_div(n, nbx)));
 }
 
 int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw, int k,
@@ -2584,10 +2576,11 @@ int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw
     const char *pname = profile ? "gram" : nullptr;
     const char *rname = profile ? "gram_reduce" : nullptr;
     const double gbytes = 8.0 * (double)n * (m + k);
-    int rows = 0, nbx = 0;
+    int nbx = 0;
     if (m <= 8 && k <= 8) {
         // register-blocked path for the small blocks of the orthonormalisation
-        nbx = gram_ranges(n, std::min(ceil_div(n, 4 * kBlock), 512), mk, partial_cap, 1, &rows);
+        nbx = gram_ranges(n, std::min(ceil_div(n, 4 * kBlock), 512), mk, partial_cap);
+        const int rows = ceil_div(n, nbx);
         if (!partial) partial = partial_buffer((size_t)nbx * mk);
         {
             ProfScope prof(pname, gbytes);
@@ -2640,7 +2633,7 @@ int gram_impl(int n, const double *V, long ldv, int m, const double *W, long ldw
         g.longer = 1;
         want = other;
     }
-    nbx = gram_ranges(n, want, mk, partial_cap, 1, &rows);
+    nbx = gram_ranges(n, want, mk, partial_cap);
     if (!partial) partial = partial_buffer((size_t)nbx * mk);
     {
         ProfScope prof(pname, gbytes);
