@@ -922,7 +922,7 @@ static void op_mv_lincomb(void **x, void **y, GCGE_INT *start, GCGE_INT *end, do
     if (m <= 0) fail_msg("MultiVecLinearComb: empty input range");
     work_vec(0, (double)m * k, Y->n);  // one axpby per coefficient (src/gcge_ops.c:190-221)
     std::vector<double> packed;
-    lincomb_pack(a, lda, m, k, packed);
+    lincomb_pack(a, lda, Y->n, m, k, packed);
     double *d_C = small_buffer(packed.size() + kLcSlack);
     upload_async(d_C, packed.data(), packed.size() * sizeof(double));
     lincomb_dev(Y->n, col_ptr(X, start[0]), X->ld, m, d_C, beta, col_ptr(Y, start[1]), Y->ld, k);
@@ -939,7 +939,7 @@ static int ext_lincomb_in_place(void **v, GCGE_INT in, GCGE_INT m, const GCGE_DO
     // the reference's work for the combination and the copy back
     work_vec(0, (double)m * k + k, X->n);
     std::vector<double> packed;
-    lincomb_pack(a, lda, m, k, packed);
+    lincomb_pack(a, lda, X->n, m, k, packed);
     double *d_C = small_buffer(packed.size() + kLcSlack);
     upload_async(d_C, packed.data(), packed.size() * sizeof(double));
     lincomb_dev(X->n, col_ptr(X, in), X->ld, m, d_C, 0.0, col_ptr(X, out), X->ld, k);

@@ -212,7 +212,7 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
 // Y's columns may overlap V's (one block of columns, same rows and leading
 // dimension) for the shapes lincomb_in_place_ok accepts, beta = 0.
 constexpr size_t kLcSlack = 8 * 8 * 64 + 2 * 256;
-void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &out);
+void lincomb_pack(const double *C, int ldc, int n, int m, int k, std::vector<double> &out);
 void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
                  long ldy, int k);
 bool lincomb_in_place_ok(int m, int k);

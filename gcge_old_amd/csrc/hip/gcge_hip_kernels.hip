@@ -1572,6 +1572,51 @@ __global__ __launch_bounds__(kBlock, 4 * NJ + NQ <= 12 ? 4 : 2) void k_lincomb(
     for (int j = 0; j < NQ; ++j) put(16 * NJ + 4 * j + kk, quad[0][j], quad[1][j]);
 }
 
+// 9 to 16 output columns from many input columns on large meshes
+// (lincomb_tall): bound by HBM (8 n (m + k) bytes).  A wavefront owns 64 rows,
+// four row tiles of 8-byte loads, and reads the coefficients of a step (one tile
+// in operand order) itself, so no wave waits for another's loads.  Whole calls
+// against k_lincomb at n = 2 048 383: 300 -> 9 columns 1012 -> 971 us, 300 -> 16
+// 1079 -> 1025 (5.05 TB/s), 200 -> 12 718 -> 697.
+__global__ __launch_bounds__(kBlock) void k_lincomb_tall(int n, const double *__restrict__ V, long ldv, int m,
+                                                         const double *__restrict__ Cp, double beta,
+                                                         double *__restrict__ Y, long ldy, int k)
+{
+    const int lane = threadIdx.x % kWave, kk = lane / 16, li = lane % 16;
+    const int r0 = (blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave) * 64;
+    if (r0 >= n) return;
+    gcge_double4 acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] = gcge_double4{0.0, 0.0, 0.0, 0.0};
+    for (int m0 = 0; m0 < m; m0 += 4) {
+        const bool in = m0 + kk < m;
+        const double a = Cp[(long)m0 * 16 + lane];
+        double b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = r0 + 16 * q + li;
+            b[q] = in && r < n ? V[(long)(m0 + kk) * ldv + r] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b[q], acc[q], 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int j = kk + 4 * v, r = r0 + 16 * q + li;
+            if (j < k && r < n) {
+                double *y = Y + (long)j * ldy + r;
+                *y = beta == 0.0 ? acc[q][v] : beta * (*y) + acc[q][v];
+            }
+        }
+}
+
+// from 2^20 rows and 192 input columns, where it is never the slower one (n = 1
+// 092 727, 300 -> 16 555 against 544 us, 200 -> 16 390 against 390, 160 -> 9 286
+// against 302; n = 357 911, 300 -> 9 183 against 210)
+inline bool lincomb_tall(int n, int m, int k) { return k > 8 && k <= 16 && m >= 192 && n >= 1 << 20; }
+
 // Few input columns (lincomb_few): bound by HBM (8 n (m + k) bytes; Y read too
 // for beta != 0), where a wave of k_lincomb has little to do for its rows and
 // k_lincomb_few loads less than the matrix products' whole stages.  A thread
@@ -1663,9 +1708,10 @@ void launch_lincomb_few(int n, const double *V, long ldv, int m, const double *d
 struct LcShape {
     int groups, cols, nj, nq;
 };
-inline LcShape lincomb_shape(int k)
+inline LcShape lincomb_shape(int n, int m, int k)
 {
     LcShape s;
+    if (lincomb_tall(n, m, k)) return {1, k, 1, 0};
     s.groups = (k + kLcCols - 1) / kLcCols;
     s.cols = (k + s.groups - 1) / s.groups;
     s.nj = s.cols / 16;
@@ -1699,7 +1745,7 @@ void launch_lincomb_q(int nq, dim3 grid, int n, const double *V, long ldv, int m
 void launch_lincomb(int n, const double *V, long ldv, int m, const double *d_C, double beta, double *Y,
                     long ldy, int k)
 {
-    const LcShape s = lincomb_shape(k);
+    const LcShape s = lincomb_shape(n, m, k);
     const dim3 grid((n + 127) / 128, s.groups);
 #define GCGE_LC(NJ) \
     case NJ: launch_lincomb_q<NJ>(s.nq, grid, n, V, ldv, m, d_C, beta, Y, ldy, k, s.cols); break
@@ -2676,7 +2722,7 @@ void gram(int n, const double *V, long ldv, int m, const double *W, long ldw, in
 // column group, step of 4 input columns, and tile (4 x 16, output column
 // fastest) or quad (4 x 4), zeros past m and k.  Few input columns: column by
 // column, zeros past m.  For the library comparison: row by row.
-void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &out)
+void lincomb_pack(const double *C, int ldc, int n, int m, int k, std::vector<double> &out)
 {
     if (use_blas(m, k)) {
         out.resize((size_t)m * k);
@@ -2693,7 +2739,7 @@ void lincomb_pack(const double *C, int ldc, int m, int k, std::vector<double> &o
             for (int i = 0; i < m; ++i) out[(size_t)j * M + i] = C[(size_t)j * ldc + i];
         return;
     }
-    const LcShape s = lincomb_shape(k);
+    const LcShape s = lincomb_shape(n, m, k);
     const int steps = ceil_div(m, 4), per_step = s.nj * kWave + s.nq * 16;
     out.assign((size_t)s.groups * steps * per_step, 0.0);
     static_assert(kLcSlack >= kLcSteps * kLcCols / 16 * kWave + 2 * kBlock, "one stage, rounded up");
@@ -2741,6 +2787,12 @@ void lincomb_dev(int n, const double *V, long ldv, int m, const double *d_C, dou
         const int least = blocks >= cus ? 4 * m : std::max(4, m);
         const int parts = apart ? std::max(1, std::min(k / least, 4 * cus / blocks)) : 1;
         launch_lincomb_few(n, V, ldv, m, d_C, beta, Y, ldy, k, ceil_div(k, std::max(parts, ceil_div(k, kLcCols))));
+        return;
+    }
+    if (lincomb_tall(n, m, k)) {
+        hipLaunchKernelGGL(k_lincomb_tall, dim3(ceil_div(n, 256)), dim3(kBlock), 0, state().stream, n, V, ldv, m,
+                           d_C, beta, Y, ldy, k);
+        HIP_CHECK(hipGetLastError());
         return;
     }
     launch_lincomb(n, V, ldv, m, d_C, beta, Y, ldy, k);

@@ -250,3 +250,30 @@ def test_element_gradient_reported_bytes(two_blocks):
     lib.GCGE_HIP_ProfileReset()
     assert count.value == 1
     assert moved.value == 8.0 * ((2 if two_blocks else 1) * k * (E - 1) ** 3 + E ** 3)
+
+
+@pytest.mark.parametrize("n,m,k", [(1 << 20, 192, 9), (1048579, 193, 16), (1100001, 300, 13), ((1 << 20) - 1, 193, 12),
+                                   (1048579, 191, 12)])
+def test_linear_comb_tall(n, m, k):
+    """Both sides of the sizes from which 9 to 16 columns have their own waves
+    of 64 rows; a rest of rows and of input columns, beta, and over the input.
+    Eight distinct input columns in turn, so the reference folds C."""
+    rng = np.random.default_rng(m + k)
+    base, C = rng.standard_normal((n, 8)), np.asfortranarray(rng.standard_normal((m, k)))
+    Y0 = rng.standard_normal((n, k))
+    fold = lambda M: np.stack([M[c::8].sum(0) for c in range(8)])
+    bound = np.abs(base) @ fold(np.abs(C))
+    dV, dY = DeviceMultiVec(n, m + 1), DeviceMultiVec.from_host(Y0)
+    for c in range(0, m, 8):
+        dV.set(np.ascontiguousarray(base[:, :min(8, m - c)]), c)
+    dV.set(np.full((n, 1), np.nan), m)
+    lib = _native.hip()
+    print(f"linear combination n={n} m={m} k={k}", flush=True)
+    lib.GCGE_HIP_LinearComb(dV.handle, 0, m, _native.as_dptr(C), m, -1.5, dY.handle, 0, k)
+    got = dY.get()
+    want = base @ fold(C) - 1.5 * Y0
+    assert np.all(np.abs(got - want) <= 2 * (m + 2) * EPS * (bound + 1.5 * np.abs(Y0)))
+    lib.GCGE_HIP_LinearComb(dV.handle, 0, m, _native.as_dptr(C), m, 0.0, dY.handle, 0, k)
+    lib.GCGE_HIP_LinearComb(dV.handle, 0, m, _native.as_dptr(C), m, 0.0, dV.handle, 3, k)
+    np.testing.assert_array_equal(dV.get(3, k), dY.get())
+    assert np.all(np.abs(dY.get() - base @ fold(C)) <= 2 * (m + 2) * EPS * bound)
