@@ -17,7 +17,8 @@
 //               with a deterministic second-pass reduction.
 //   lincomb     Y = beta Y + V C on the matrix cores: a wavefront owns 32 rows
 //               and all output columns of a group, V goes straight to
-//               registers, the coefficients through LDS.
+//               registers, the coefficients through LDS; own kernels for few
+//               input columns and for 9 to 16 columns of large meshes.
 //   axpby/swap/random/coldots/residual/bcg_*: streaming kernels.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
